@@ -1079,6 +1079,7 @@ struct csrst_warmstart {
         DBuf<uint8_t> dcls;
         DBuf<double> b, phi, pstar, part;
         DBuf<double> pprev, rprev;     // the previous iterate and its residual (two-direction step)
+        DBuf<float> dir;               // the network's direction as a level-0 array
         DBuf<bf16> pairIn;             // [maxBatch][H][W] r / rms(r)
         DBuf<float> pairTgt;           // [maxBatch][H][W] e / rms(e)
     } loop;
@@ -1328,18 +1329,72 @@ void upload_input(csrst_warmstart *u, const float *rho, int B, float scale)
 
 constexpr int kRed = 256;      // blocks of the fixed-order reductions
 
-// r * inv as bf16 network input, zero off the unknowns
-__global__ void k_res_in(const double *res, const uint8_t *act, bf16 *in, size_t n, double inv)
+// The multigrid's arrays are in its own column order (pmg::Level::at), the
+// network's images row-major: these kernels go between the two, a 32 x 32 tile per workgroup
+// through LDS, so that both sides are read and written along their rows.
+constexpr int kT = pmg::kTile;
+
+// level value get(k) at the unknowns (0 elsewhere) to the image put(p, v)
+template <class Get, class Put>
+__device__ __forceinline__ void level_to_image(const pmg::Level &L, Get get, Put put)
 {
-    const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (k < n) in[k] = act[k] ? f2bf((float)(res[k] * inv)) : (bf16)0;
+    __shared__ float t[kT][kT + 1];
+    const int i0 = blockIdx.x * kT, j0 = blockIdx.y * kT, a = threadIdx.x % kT, row = threadIdx.x / kT;
+    for (int r = row; r < kT; r += kB / kT) {
+        const int i = i0 + r, j = j0 + a;
+        const size_t k = L.at(i, j);
+        t[r][a] = i < L.nx && j < L.ny && L.act[k] ? get(k) : 0.f;
+    }
+    __syncthreads();
+    for (int r = row; r < kT; r += kB / kT) {
+        const int i = i0 + a, j = j0 + r;
+        if (i < L.nx && j < L.ny) put((size_t)j * L.nx + i, t[a][r]);
+    }
+}
+
+// r * inv as bf16 network input, zero off the unknowns
+__global__ void __launch_bounds__(kB) k_res_in(pmg::Level L, bf16 *in, double inv)
+{
+    level_to_image(L, [&](size_t k) { return (float)(L.res[k] * inv); }, [&](size_t p, float v) { in[p] = f2bf(v); });
 }
 
 // (pstar - phi) * inv as float target, zero off the unknowns
-__global__ void k_err_tgt(const double *pstar, const double *phi, const uint8_t *act, float *t, size_t n, double inv)
+__global__ void __launch_bounds__(kB) k_err_tgt(pmg::Level L, const double *pstar, float *t, double inv)
 {
-    const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (k < n) t[k] = act[k] ? (float)((pstar[k] - phi[k]) * inv) : 0.f;
+    level_to_image(L, [&](size_t k) { return (float)((pstar[k] - L.phi[k]) * inv); }, [&](size_t p, float v) { t[p] = v; });
+}
+
+// the network's output image as a level array
+__global__ void __launch_bounds__(kB) k_dir_in(pmg::Level L, const float *img, float *c)
+{
+    __shared__ float t[kT][kT + 1];
+    const int i0 = blockIdx.x * kT, j0 = blockIdx.y * kT, a = threadIdx.x % kT, row = threadIdx.x / kT;
+    for (int r = row; r < kT; r += kB / kT) {
+        const int i = i0 + a, j = j0 + r;
+        t[r][a] = i < L.nx && j < L.ny ? img[(size_t)j * L.nx + i] : 0.f;
+    }
+    __syncthreads();
+    for (int r = row; r < kT; r += kB / kT) {
+        const int i = i0 + r, j = j0 + a;
+        if (i < L.nx && j < L.pitch) c[L.at(i, j)] = t[a][r];
+    }
+}
+
+dim3 tile_grid(const pmg::Level &L) { return dim3((L.nx + kT - 1) / kT, (L.pitch + kT - 1) / kT); }
+
+// c . A c's row k: the level's 5-point operator with the unknowns' couplings
+// only, as the multigrid applies it
+__device__ __forceinline__ double apply_dir(const pmg::Level &L, const float *c, size_t k)
+{
+    const int i = (int)(k / L.pitch), q = (int)(k % L.pitch), N = 64 * L.lane;
+    const int j = q / N * N + (q % 128) / 2 * L.lane + 2 * (q % N / 128) + (q & 1);   // row_pos inverted
+    double sx = 0.0, sy = 0.0;
+    if (i > 0 && L.act[k - L.pitch]) sx += c[k - L.pitch];
+    if (i + 1 < L.nx && L.act[k + L.pitch]) sx += c[k + L.pitch];
+    const size_t d = L.at(i, j > 0 ? j - 1 : j), u = L.at(i, j + 1 < L.ny ? j + 1 : j);
+    if (j > 0 && L.act[d]) sy += c[d];
+    if (j + 1 < L.ny && L.act[u]) sy += c[u];
+    return 2.0 * (L.cx + L.cy) * (double)c[k] - L.cx * sx - L.cy * sy;
 }
 
 __device__ __forceinline__ void block_sum2(double &a, double &b, double *part)
@@ -1361,27 +1416,6 @@ __device__ __forceinline__ void block_sum2(double &a, double &b, double *part)
     }
 }
 
-// partial sums of c . r and c . A c over the unknowns (A the level's 5-point
-// operator with the unknowns' couplings only, as the multigrid applies it)
-__global__ void __launch_bounds__(kB) k_step_dots(pmg::Level L, const float *c, double *part)
-{
-    double cr = 0.0, cac = 0.0;
-    const size_t n = (size_t)L.nx * L.ny;
-    for (size_t k = (size_t)blockIdx.x * kB + threadIdx.x; k < n; k += (size_t)gridDim.x * kB) {
-        if (!L.act[k]) continue;
-        const int i = (int)(k % L.nx), j = (int)(k / L.nx);
-        const double ck = c[k];
-        double sx = 0.0, sy = 0.0;
-        if (i > 0 && L.act[k - 1]) sx += c[k - 1];
-        if (i + 1 < L.nx && L.act[k + 1]) sx += c[k + 1];
-        if (j > 0 && L.act[k - L.nx]) sy += c[k - L.nx];
-        if (j + 1 < L.ny && L.act[k + L.nx]) sy += c[k + L.nx];
-        cr += ck * L.res[k];
-        cac += ck * (2.0 * (L.cx + L.cy) * ck - L.cx * sx - L.cy * sy);
-    }
-    block_sum2(cr, cac, part);
-}
-
 // partial sums of (pstar - phi)^2 over the unknowns (second slot unused)
 __global__ void __launch_bounds__(kB) k_err_sumsq(const double *pstar, const double *phi, const uint8_t *act, size_t n,
                                                  double *part)
@@ -1395,28 +1429,26 @@ __global__ void __launch_bounds__(kB) k_err_sumsq(const double *pstar, const dou
     block_sum2(s, z, part);
 }
 
-// The two-direction step: partial sums over the unknowns of c.Ac, c.Ad, d.Ad,
-// c.r, d.r with d = phi - pprev (the previous iteration's change) and
-// A d = rprev - r; c may be null (d alone).  Five doubles per block.
+// The step's sums: partial sums over the unknowns of c.Ac, c.Ad, d.Ad, c.r,
+// d.r with d = phi - pprev (the previous iteration's change) and A d = rprev -
+// r; c or pprev may be null (their sums are zero).  Five doubles per block.
 __global__ void __launch_bounds__(kB) k_step_dots5(pmg::Level L, const float *c, const double *pprev,
                                                    const double *rprev, double *part)
 {
     __shared__ double sh[5][kB];
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    const size_t n = (size_t)L.nx * L.ny;
+    const size_t n = (size_t)L.nx * L.pitch;
     for (size_t k = (size_t)blockIdx.x * kB + threadIdx.x; k < n; k += (size_t)gridDim.x * kB) {
         if (!L.act[k]) continue;
-        const double r = L.res[k], d = L.phi[k] - pprev[k], ad = rprev[k] - r;
-        double ck = 0.0, ack = 0.0;
+        const double r = L.res[k];
+        double ck = 0.0, ack = 0.0, d = 0.0, ad = 0.0;
+        if (pprev) {
+            d = L.phi[k] - pprev[k];
+            ad = rprev[k] - r;
+        }
         if (c) {
-            const int i = (int)(k % L.nx), j = (int)(k / L.nx);
             ck = c[k];
-            double sx = 0.0, sy = 0.0;
-            if (i > 0 && L.act[k - 1]) sx += c[k - 1];
-            if (i + 1 < L.nx && L.act[k + 1]) sx += c[k + 1];
-            if (j > 0 && L.act[k - L.nx]) sy += c[k - L.nx];
-            if (j + 1 < L.ny && L.act[k + L.nx]) sy += c[k + L.nx];
-            ack = 2.0 * (L.cx + L.cy) * ck - L.cx * sx - L.cy * sy;
+            ack = apply_dir(L, c, k);
         }
         s[0] += ck * ack;
         s[1] += ck * ad;
@@ -1436,47 +1468,68 @@ __global__ void __launch_bounds__(kB) k_step_dots5(pmg::Level L, const float *c,
     if (threadIdx.x < 5) part[5 * blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-__global__ void k_sum5_final(double *part, int nb)
+// The step's coefficients from the kRed blocks' sums, on the device (the host
+// would only hold the stream up for them): the energy-norm minimiser over
+// span{c, d}, a 2 x 2 system, or over the one direction that is there and not
+// degenerate.  coef = (alpha, beta).
+__global__ void __launch_bounds__(kB) k_step_coef(const double *part, double *coef)
 {
-    if (threadIdx.x >= 5 || blockIdx.x != 0) return;
-    double a = 0.0;
-    for (int k = 0; k < nb; ++k) a += part[5 * k + threadIdx.x];
-    part[5 * nb + threadIdx.x] = a;
+    static_assert(kRed == kB, "one partial per thread");
+    __shared__ double sh[5][kB];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) sh[q][threadIdx.x] = part[5 * threadIdx.x + q];
+    __syncthreads();
+    for (int o = kB / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x) return;
+    const double cac = sh[0][0], cad = sh[1][0], dad = sh[2][0], cr = sh[3][0], dr = sh[4][0];
+    double alpha = 0.0, beta = 0.0;
+    const bool hc = cac > 0, hd = dad > 0;
+    const double det = cac * dad - cad * cad;
+    if (hc && hd && det > 1e-12 * cac * dad) {
+        alpha = (cr * dad - cad * dr) / det;
+        beta = (cac * dr - cad * cr) / det;
+    } else if (hc) {
+        alpha = cr / cac;
+    } else if (hd) {
+        beta = dr / dad;
+    }
+    if (!isfinite(alpha) || !isfinite(beta)) alpha = beta = 0.0;
+    coef[0] = alpha;
+    coef[1] = beta;
 }
 
-// phi += alpha c + beta (phi - pprev) on the unknowns; pprev, rprev take the
-// iterate and residual before the step
-__global__ void k_update2(pmg::Level L, const float *c, double alpha, double beta, double *pprev, double *rprev)
+// phi += alpha c + beta (phi - pprev) on the unknowns; pprev, rprev (if any)
+// take the iterate and residual before the step
+__global__ void k_step_update(pmg::Level L, const float *c, const double *coef, double *pprev, double *rprev)
 {
     const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (k >= (size_t)L.nx * L.ny) return;
-    if (!L.act[k]) {
-        pprev[k] = 0.0;
-        rprev[k] = 0.0;
-        return;
+    if (k >= (size_t)L.nx * L.pitch || !L.act[k]) return;
+    const double ph = L.phi[k];
+    double v = c ? ph + coef[0] * (double)c[k] : ph;
+    if (pprev) {
+        v += coef[1] * (ph - pprev[k]);
+        pprev[k] = ph;
+        rprev[k] = L.res[k];
     }
-    const double ph = L.phi[k], d = ph - pprev[k];
-    pprev[k] = ph;
-    rprev[k] = L.res[k];
-    L.phi[k] = ph + (c ? alpha * (double)c[k] : 0.0) + beta * d;
+    L.phi[k] = v;
 }
 
-__global__ void k_sum2_final(double *part, int nb)
+// the first of the kRed blocks' sums, on one workgroup
+__global__ void __launch_bounds__(kB) k_sum2_final(double *part)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double a = 0.0, b = 0.0;
-    for (int k = 0; k < nb; ++k) {
-        a += part[2 * k];
-        b += part[2 * k + 1];
+    __shared__ double sh[kB];
+    sh[threadIdx.x] = part[2 * threadIdx.x];
+    __syncthreads();
+    for (int o = kB / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
     }
-    part[2 * nb] = a;
-    part[2 * nb + 1] = b;
-}
-
-__global__ void k_axpy_act(pmg::Level L, const float *c, double alpha)
-{
-    const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (k < (size_t)L.nx * L.ny && L.act[k]) L.phi[k] += alpha * (double)c[k];
+    if (threadIdx.x == 0) part[2 * kRed] = sh[0];
 }
 
 __global__ void k_copy_d(double *dst, const double *src, size_t n)
@@ -1517,89 +1570,54 @@ void loop_grid(csrst_warmstart *u, double hx, double hy, const uint8_t *cls)
     Lp.ready = false;
     Lp.cls.assign(cls, cls + n);
     Lp.dcls.alloc(n);
-    Lp.b.alloc(n); Lp.phi.alloc(n); Lp.pstar.alloc(n); Lp.part.alloc(5 * kRed + 5);
-    Lp.pprev.alloc(n); Lp.rprev.alloc(n);
+    Lp.b.alloc(n); Lp.phi.alloc(n); Lp.part.alloc(5 * kRed + 2);
     HU_CHECK(hipMemcpyAsync(Lp.dcls.p, cls, n, hipMemcpyHostToDevice, u->s));
     Lp.mg.setup(u->W, u->H, hx, hy, Lp.dcls.p, u->s);
+    const size_t nl = Lp.mg.level0_size();
+    Lp.pstar.alloc(nl); Lp.pprev.alloc(nl); Lp.rprev.alloc(nl); Lp.dir.alloc(nl);
     Lp.hx = hx; Lp.hy = hy; Lp.unknowns = unk;
     Lp.ready = true;
 }
 
-// the two sums of the last k_step_dots / k_err_sumsq launch on the host
-void loop_sums(csrst_warmstart *u, double &a, double &b)
+// the sum of the last k_err_sumsq launch on the host
+double loop_sum(csrst_warmstart *u)
 {
     auto &Lp = u->loop;
-    k_sum2_final<<<1, 1, 0, u->s>>>(Lp.part.p, kRed);
+    k_sum2_final<<<1, kB, 0, u->s>>>(Lp.part.p);
     HU_LAUNCH_CHECK();
-    double h[2];
-    HU_CHECK(hipMemcpyAsync(h, Lp.part.p + 2 * kRed, sizeof h, hipMemcpyDeviceToHost, u->s));
+    double h = 0.0;
+    HU_CHECK(hipMemcpyAsync(&h, Lp.part.p + 2 * kRed, sizeof h, hipMemcpyDeviceToHost, u->s));
     HU_CHECK(hipStreamSynchronize(u->s));
-    a = h[0];
-    b = h[1];
+    return h;
 }
 
-// The network's step at the current iterate; rn = ||r|| from resnorm().
-void loop_correct(csrst_warmstart *u, double rn)
+// The step at the current iterate, rn = ||r|| from resnorm(): over the
+// network's direction (useNet), the previous iteration's change (usePrev), or
+// both.  first: no previous iterate yet (d = 0).
+void loop_step(csrst_warmstart *u, double rn, bool useNet, bool usePrev, bool first)
 {
     auto &Lp = u->loop;
     const pmg::Level &L0 = Lp.mg.level0();
-    const size_t n = (size_t)u->H * u->W;
+    const size_t nl = Lp.mg.level0_size();
     const double rms = rn / std::sqrt((double)Lp.unknowns);
     if (!(rms > 0)) return;
-    plan(u, 1);
-    k_res_in<<<nb(n), kB, 0, u->s>>>(L0.res, L0.act, u->ptr(u->A[0]), n, 1.0 / rms);
-    forward(u, 1);
-    k_step_dots<<<kRed, kB, 0, u->s>>>(L0, u->outf.p, Lp.part.p);
-    double cr = 0, cac = 0;
-    loop_sums(u, cr, cac);
-    if (cac > 0 && std::isfinite(cr / cac)) {
-        k_axpy_act<<<nb(n), kB, 0, u->s>>>(L0, u->outf.p, cr / cac);
-        HU_LAUNCH_CHECK();
-    }
-}
-
-// The step over the network's direction (useNet) and the previous iteration's
-// change: the energy-norm minimiser over span{c, d}, a 2 x 2 system (one
-// direction when the other is absent or degenerate).  first: no previous
-// iterate yet (d = 0).
-void loop_step2(csrst_warmstart *u, double rn, bool useNet, bool first)
-{
-    auto &Lp = u->loop;
-    const pmg::Level &L0 = Lp.mg.level0();
-    const size_t n = (size_t)u->H * u->W;
-    const double rms = rn / std::sqrt((double)Lp.unknowns);
-    if (!(rms > 0)) return;
-    if (first) {
-        k_copy_d<<<nb(n), kB, 0, u->s>>>(Lp.pprev.p, L0.phi, n);
-        k_copy_d<<<nb(n), kB, 0, u->s>>>(Lp.rprev.p, L0.res, n);
+    if (usePrev && first) {
+        k_copy_d<<<nb(nl), kB, 0, u->s>>>(Lp.pprev.p, L0.phi, nl);
+        k_copy_d<<<nb(nl), kB, 0, u->s>>>(Lp.rprev.p, L0.res, nl);
     }
     const float *c = nullptr;
     if (useNet) {
         plan(u, 1);
-        k_res_in<<<nb(n), kB, 0, u->s>>>(L0.res, L0.act, u->ptr(u->A[0]), n, 1.0 / rms);
+        k_res_in<<<tile_grid(L0), kB, 0, u->s>>>(L0, u->ptr(u->A[0]), 1.0 / rms);
         forward(u, 1);
-        c = u->outf.p;
+        k_dir_in<<<tile_grid(L0), kB, 0, u->s>>>(L0, u->outf.p, Lp.dir.p);
+        c = Lp.dir.p;
     }
-    k_step_dots5<<<kRed, kB, 0, u->s>>>(L0, c, Lp.pprev.p, Lp.rprev.p, Lp.part.p);
-    k_sum5_final<<<1, 64, 0, u->s>>>(Lp.part.p, kRed);
-    HU_LAUNCH_CHECK();
-    double h[5];
-    HU_CHECK(hipMemcpyAsync(h, Lp.part.p + 5 * kRed, sizeof h, hipMemcpyDeviceToHost, u->s));
-    HU_CHECK(hipStreamSynchronize(u->s));
-    const double cac = h[0], cad = h[1], dad = h[2], cr = h[3], dr = h[4];
-    double alpha = 0.0, beta = 0.0;
-    const bool hc = c && cac > 0, hd = dad > 0;
-    const double det = cac * dad - cad * cad;
-    if (hc && hd && det > 1e-12 * cac * dad) {
-        alpha = (cr * dad - cad * dr) / det;
-        beta = (cac * dr - cad * cr) / det;
-    } else if (hc) {
-        alpha = cr / cac;
-    } else if (hd) {
-        beta = dr / dad;
-    }
-    if (!std::isfinite(alpha) || !std::isfinite(beta)) alpha = beta = 0.0;
-    k_update2<<<nb(n), kB, 0, u->s>>>(L0, c, alpha, beta, Lp.pprev.p, Lp.rprev.p);
+    double *pp = usePrev ? Lp.pprev.p : nullptr, *rp = usePrev ? Lp.rprev.p : nullptr;
+    double *coef = Lp.part.p + 5 * kRed;
+    k_step_dots5<<<kRed, kB, 0, u->s>>>(L0, c, pp, rp, Lp.part.p);
+    k_step_coef<<<1, kB, 0, u->s>>>(Lp.part.p, coef);
+    k_step_update<<<nb(nl), kB, 0, u->s>>>(L0, c, coef, pp, rp);
     HU_LAUNCH_CHECK();
 }
 
@@ -1798,8 +1816,7 @@ int csrst_warmstart_solve(csrst_warmstart *u, double hx, double hy, const uint8_
         const double target = tol * (bn > 0 ? bn : 1.0);
         int cyc = 0, flat = 0;
         while (r > target && cyc < maxit && flat < 3) {
-            if (mode == 1 || (mode == 2 && cyc == 0)) loop_correct(u, r);
-            else if (mode >= 3) loop_step2(u, r, mode == 3, cyc == 0);
+            if (mode >= 3 || mode == 1 || (mode == 2 && cyc == 0)) loop_step(u, r, mode != 4, mode >= 3, cyc == 0);
             Lp.mg.cycle();
             ++cyc;
             const double rn = Lp.mg.resnorm();
@@ -1838,6 +1855,7 @@ int csrst_warmstart_train_iterates(csrst_warmstart *u, double hx, double hy, con
         Lp.pairIn.alloc(std::max(Lp.pairIn.n, (size_t)MB * n));
         Lp.pairTgt.alloc(std::max(Lp.pairTgt.n, (size_t)MB * n));
         const pmg::Level &L0 = Lp.mg.level0();
+        const size_t nl = Lp.mg.level0_size();
         int slot = 0, used = 0, nsteps = 0;
         double lsum = 0.0;
         for (int i = 0; i < nrhs; ++i) {
@@ -1853,18 +1871,16 @@ int csrst_warmstart_train_iterates(csrst_warmstart *u, double hx, double hy, con
                 flat = rn > 0.95 * r ? flat + 1 : 0;
                 r = rn;
             }
-            k_copy_d<<<nb(n), kB, 0, u->s>>>(Lp.pstar.p, L0.phi, n);
+            k_copy_d<<<nb(nl), kB, 0, u->s>>>(Lp.pstar.p, L0.phi, nl);
             Lp.mg.begin(Lp.b.p, Lp.phi.p);
             r = Lp.mg.resnorm();
             for (int k = 0; k < kmax && r > 1e-12 * bn; ++k) {
-                k_err_sumsq<<<kRed, kB, 0, u->s>>>(Lp.pstar.p, L0.phi, L0.act, n, Lp.part.p);
-                double e2 = 0, z = 0;
-                loop_sums(u, e2, z);
+                k_err_sumsq<<<kRed, kB, 0, u->s>>>(Lp.pstar.p, L0.phi, L0.act, nl, Lp.part.p);
+                const double e2 = loop_sum(u);
                 const double rr = r / std::sqrt((double)Lp.unknowns), re = std::sqrt(e2 / (double)Lp.unknowns);
                 if (rr > 0 && re > 0) {
-                    k_res_in<<<nb(n), kB, 0, u->s>>>(L0.res, L0.act, Lp.pairIn.p + (size_t)slot * n, n, 1.0 / rr);
-                    k_err_tgt<<<nb(n), kB, 0, u->s>>>(Lp.pstar.p, L0.phi, L0.act, Lp.pairTgt.p + (size_t)slot * n, n,
-                                                       1.0 / re);
+                    k_res_in<<<tile_grid(L0), kB, 0, u->s>>>(L0, Lp.pairIn.p + (size_t)slot * n, 1.0 / rr);
+                    k_err_tgt<<<tile_grid(L0), kB, 0, u->s>>>(L0, Lp.pstar.p, Lp.pairTgt.p + (size_t)slot * n, 1.0 / re);
                     HU_LAUNCH_CHECK();
                     if (++slot == MB) {
                         lsum += loop_train(u, slot, lr);
@@ -1873,7 +1889,7 @@ int csrst_warmstart_train_iterates(csrst_warmstart *u, double hx, double hy, con
                         slot = 0;
                     }
                 }
-                if (inloop) loop_correct(u, r);
+                if (inloop) loop_step(u, r, true, false, false);
                 Lp.mg.cycle();
                 r = Lp.mg.resnorm();
             }
