@@ -90,6 +90,23 @@ def test_charge_diff_continuity(gpu, order):
     assert np.abs(diff + dt * div).max() < 1e-12 * scale
 
 
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("n", [1, 63, 65, 20312, 20313, 60000])
+def test_small_and_sorted_deposits_bitwise(gpu, order, n):
+    """Particle counts around a wavefront, around the line between the node
+    scan and the sorted deposit (130e6 item-node pairs: 20312 trajectories on
+    40 x 40 nodes), and runs of hundreds of contributions per node; the
+    repeated call takes the first one's workspace."""
+    dx, dt = (0.7, 1.3), 0.37
+    box, org = (-6, -6, 40, 40), (0.0, 0.0)
+    oldR, R, q = trajectories(n, order + n)
+    for comp in (0, 1):
+        ref = O.deposit(order, comp, box, org, dx, dt, oldR, R, q)
+        for _ in range(2):
+            assert same(SF.getCurrentDensity(order, comp, box, org, dx, dt, oldR, R, q), ref), "comp %d" % comp
+    assert same(SF.getChargeDensity(order, box, org, dx, R, q), O.charge_density(order, box, org, dx, R, q))
+
+
 def test_patch_overflow_is_reported(gpu):
     oldR, R, q = trajectories(50, 1)
     with pytest.raises(CsrstError) as e:
