@@ -504,8 +504,7 @@ __device__ __forceinline__ void seg_s2_gauss(pm::SegCurrent<T> &o, int comp, T t
 }
 
 constexpr int kRun = 4;              // consecutive particles per vector load (16 B of FP32, 32 B of FP64)
-constexpr int kPPT = 4;              // particles per thread: one run of kRun consecutive sorted particles
-constexpr int kChunk = kB * kPPT;    // 1024 particles per workgroup
+constexpr int kPPT = kRun;           // particles per thread: one run of consecutive sorted particles
 constexpr int kTW = 64, kTH = 32;    // LDS accumulation tile (nodes)
 constexpr int kSlots = 2;            // register accumulation slots per lane (one stencil anchor each)
 constexpr int kMaxSub = 8;           // sort key: at most 2^8 x 2^8 bins per cell
@@ -516,6 +515,16 @@ template <class T>
 struct alignas(16) Run {
     T v[kRun];
 };
+template <class T>
+__device__ __forceinline__ void load_run(const T *a, int k0, int n, T (&o)[1])
+{
+    o[0] = k0 < n ? a[k0] : T(0);
+}
+template <class T>
+__device__ __forceinline__ void store_run(T *a, int k0, int n, const T (&o)[1])
+{
+    if (k0 < n) a[k0] = o[0];
+}
 template <class T>
 __device__ __forceinline__ void load_run(const T *a, int k0, int n, T (&o)[kRun])
 {
@@ -543,16 +552,30 @@ __device__ __forceinline__ void store_run(T *a, int k0, int n, const T (&o)[kRun
     }
 }
 // shift a run down by one register and append v (keeps every index static)
-template <class T>
-__device__ __forceinline__ void rotate_in(T (&o)[kRun], T v)
+template <int N, class T>
+__device__ __forceinline__ void rotate_in(T (&o)[N], T v)
 {
 #pragma unroll
-    for (int u = 0; u < kRun - 1; ++u) o[u] = o[u + 1];
-    o[kRun - 1] = v;
+    for (int u = 0; u < N - 1; ++u) o[u] = o[u + 1];
+    o[N - 1] = v;
 }
 
-// Push of one workgroup chunk (kChunk sorted particles): thread t owns
-// particles base + kPPT t .. + kPPT - 1, so its consecutive particles share a
+// Up to this many particles a thread takes one particle (PPT = 1) and adds its
+// segments straight into the LDS tile; above, it takes a run.  The run form
+// needs 1024 particles per workgroup and ends with passes per distinct anchor,
+// so it takes 57 to 120 us however few there are; the other form's LDS atomics
+// collide on a dense bunch and cost 0.16 us per 1000 particles.  us per push,
+// bunch of 20 x 10 cells in the bend, one particle / run:
+//   FP32 S1  1e5 17/58, 7e5 64/63    S2  1e5 31/80, 3e5 73/85, 7e5 143/87
+//   FP32 S0  1e5 12/58, 1.5e6 72/78  FP64 S2  2e4 20/115, 7e5 105/141, 1.5e6 209/180
+template <class T>
+constexpr int few_particles(int order)
+{
+    return sizeof(T) == 8 ? 1000000 : order == 0 ? 1500000 : order == 1 ? 650000 : 350000;
+}
+
+// Push of one workgroup chunk (kB PPT sorted particles): thread t owns
+// particles base + PPT t .. + PPT - 1, so its consecutive particles share a
 // cell and their segment currents share stencil anchors.  Currents collect in
 // kSlots register slots per lane (one anchor each).  A segment whose anchor
 // matches neither (a run crossing a cell boundary, or a bunch moving at an
@@ -568,14 +591,14 @@ __device__ __forceinline__ void rotate_in(T (&o)[kRun], T v)
 // (c3 at 1-10 deg: the cooperative form 13-25 % faster; c2 at 1-8 deg: 2-8 %
 // slower; along x the cooperative path in the loop costs 20 %), so the step
 // times the two against each other and keeps the faster (csrst_mw_step).
-template <class T, int ORDER, int COMP, bool MISSCOOP>
+template <class T, int ORDER, int COMP, bool MISSCOOP, int PPT>
 __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3))) k_push(Parts<T> p, Fields<T> f, Geo g, PushConst<T> c, WinState *ws)
 {
     __shared__ T acc[kTH * kTW];
     __shared__ int pbox[4];          // particle cell box of the chunk (min x, min y, -max x, -max y)
     const int tid = threadIdx.x, lane = tid & 63;
-    const int base = blockIdx.x * kChunk;
-    const int kt = base + tid * kPPT;           // this thread's first particle
+    const int base = blockIdx.x * (kB * PPT);
+    const int kt = base + tid * PPT;            // this thread's first particle
     const int wx0 = ws->wx0, wy0 = ws->wy0, rx = ws->rx, ry = ws->ry;
     const vec2<T> p0 = pm::mk((T)ws->p0[0], (T)ws->p0[1]);
     const int W = f.W, H = f.H;
@@ -619,7 +642,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
     // sums 16 of node l / 4's values and a quad sum completes it, then lanes
     // 4t add node t into the tile in one step.  Called in wave-uniform control
     // flow (every lane active).
-    __shared__ T red[(kB / 64) * NN * 64];
+    __shared__ T red[PPT == 1 ? 1 : (kB / 64) * NN * 64];
     T *rw = red + (tid >> 6) * (NN * 64);
     auto coop_add = [&](bool mine0, int sI, int sJ, const T *w) {
         unsigned long long rem = __ballot(mine0);
@@ -664,10 +687,11 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
         sc.I0 += cgx; sc.J0 += cgy;   // global node of the first stencil entry
     };
     // per-wave queue of third segments: xi, xf, tau, displacement; old cell
-    __shared__ T qvAll[kB / 64][7][64];
-    __shared__ int qgAll[kB / 64][2][64];
-    T (*qv)[64] = qvAll[tid >> 6];
-    int (*qg)[64] = qgAll[tid >> 6];
+    constexpr int QW = PPT == 1 ? 1 : kB / 64;   // PPT = 1 has no queue
+    __shared__ T qvAll[QW][7][64];
+    __shared__ int qgAll[QW][2][64];
+    T (*qv)[64] = qvAll[PPT == 1 ? 0 : tid >> 6];
+    int (*qg)[64] = qgAll[PPT == 1 ? 0 : tid >> 6];
     int qn = 0;   // wave-uniform queue length
     auto drain_queue = [&]() {
         __builtin_amdgcn_wave_barrier();
@@ -691,10 +715,10 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
         for (int t = 0; t < NN; ++t) sacc[q][t] = T(0);
     }
 #pragma unroll 1
-    for (int r = 0; r < kPPT / kRun; ++r) {
-        const int k0 = kt + r * kRun;
-        int GX[kRun], GY[kRun];
-        T FX[kRun], FY[kRun], PX[kRun], PY[kRun];
+    for (int r = 0; r < 1; ++r) {
+        const int k0 = kt;
+        int GX[PPT], GY[PPT];
+        T FX[PPT], FY[PPT], PX[PPT], PY[PPT];
         load_run(p.gx, k0, p.n, GX);
         load_run(p.gy, k0, p.n, GY);
         load_run(p.fx, k0, p.n, FX);
@@ -702,7 +726,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
         load_run(p.px, k0, p.n, PX);
         load_run(p.py, k0, p.n, PY);
 #pragma unroll 1
-        for (int u = 0; u < kRun; ++u) {
+        for (int u = 0; u < PPT; ++u) {
             const bool live = k0 + u < p.n;
             const int gx0 = GX[0], gy0 = GY[0];
             const T fx0 = FX[0], fy0 = FY[0];
@@ -840,6 +864,20 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
             if (live && !oneCross) err |= 2;
             const vec2<T> delta = pm::mk(e.x - o.x, e.y - o.y);
             const int nseg = live ? xs.n - 1 : 0;
+            if constexpr (PPT == 1) {
+                // every segment straight into the LDS tile
+#pragma unroll 1
+                for (int s = 0; s < 3; ++s) {
+                    const bool act = s < nseg;
+                    if (!__any(act)) break;
+                    pm::SegCurrent<T> sc;
+                    const vec2<T> xi = sel(s == 0, xs.s[0], sel(s == 1, xs.s[1], xs.s[2]));
+                    const vec2<T> xf = sel(s == 0, xs.s[1], sel(s == 1, xs.s[2], xs.s[3]));
+                    const T tau = s == 0 ? xs.f[1] - xs.f[0] : s == 1 ? xs.f[2] - xs.f[1] : xs.f[3] - xs.f[2];
+                    seg_current(sc, xi, xf, tau, delta, gx0, gy0);
+                    if (act) lane_add(sc.I0, sc.J0, sc.w);
+                }
+            } else {
             // third segments (a push crossing a cell column and a cell row) are
             // queued and computed 64 at a time: in-line, one lane with three
             // segments makes its whole wavefront run a third segment pass
@@ -897,6 +935,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
                     lane_add(sc.I0, sc.J0, sc.w);
                 }
             }
+            }
             // ---- drift back by half a step (TETMSolver.hh:210, 265)
             if (live) {
                 const int ex2 = gx0 + (int)pm::floor_(x2), ey2 = gy0 + (int)pm::floor_(y2);
@@ -918,6 +957,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
         store_run(p.py, k0, p.n, PY);
     }
     // ---- queued third segments, then the register slots
+    if constexpr (PPT > 1) {
     if (qn) drain_queue();
 #pragma unroll 1
     for (int slot = 0; slot < kSlots; ++slot) {
@@ -935,6 +975,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
             for (int t = 0; t < NN; ++t) w[t] = slot == q ? sacc[q][t] : w[t];
         }
         coop_add(h, I, Jn, w);
+    }
     }
     // ---- chunk's particle box and error bits, then flush the tile with one
     // global atomic per nonzero node
@@ -1787,13 +1828,14 @@ void launch_push(csrst_mw *m)
 {
     mw::PushConst<T> c;
     push_consts(m, c);
-    const dim3 grid((m->n + mw::kChunk - 1) / mw::kChunk);
-    if (m->tilted)
-        hipLaunchKernelGGL((mw::k_push<T, ORDER, COMP, true>), grid, dim3(mw::kB), 0, m->s, m->parts<T>(m->partBuf),
+    auto go = [&](auto kern, int ppt) {
+        const int chunk = mw::kB * ppt;
+        hipLaunchKernelGGL(kern, dim3((m->n + chunk - 1) / chunk), dim3(mw::kB), 0, m->s, m->parts<T>(m->partBuf),
                            m->fields<T>(), m->geo, c, m->ws.p);
-    else
-        hipLaunchKernelGGL((mw::k_push<T, ORDER, COMP, false>), grid, dim3(mw::kB), 0, m->s, m->parts<T>(m->partBuf),
-                           m->fields<T>(), m->geo, c, m->ws.p);
+    };
+    if (m->n <= mw::few_particles<T>(ORDER)) go(mw::k_push<T, ORDER, COMP, false, 1>, 1);
+    else if (m->tilted) go(mw::k_push<T, ORDER, COMP, true, mw::kPPT>, mw::kPPT);
+    else go(mw::k_push<T, ORDER, COMP, false, mw::kPPT>, mw::kPPT);
 }
 
 template <class T, int COMP>

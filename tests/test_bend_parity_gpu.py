@@ -241,6 +241,41 @@ def test_production_push_vs_oracle(gpu, fp32, comp, tilt):
     assert err_p < tol[0] and err_r < tol[1] and err_j < tol[2]
 
 
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("fp32,n", [(True, 63), (True, 257), (True, 340001), (True, 1500001), (False, 999999),
+                                    (False, 1000001)])
+def test_push_forms_vs_oracle(gpu, fp32, n, order):
+    """The push takes one particle per thread up to a count and a run of them
+    above (FP32: 1.5e6, 6.5e5 and 3.5e5 for the orders 0, 1, 2; FP64: 1e6):
+    either form on uniform fields against the oracle, in the bend and at a
+    tilt, with odd counts.  A node sums up to 3e4 contributions, whose FP32
+    rounding is sqrt(3e4) 2^-24 = 1e-5 of it; momenta and positions are single
+    particles', as in test_production_push_vs_oracle."""
+    b = O.Bend(Nx=1100, Ny=120, **GEOM)
+    hx, hy = b.hr
+    R, P, Q = arc_bunch(n, 5e-3, 25.0, seed=n)
+    m = MovingWindowStep(256, 64, hx, hy, order=order, fp32=fp32, sortEvery=0, statModulus=0, **GEOM)
+    m.init_bunch(R, P, Q)
+    inf = m.info()
+    (wx0, wy0), dt = inf["pos"], inf["dt"]
+    F = np.zeros((6, m.H + 2, m.W + 2))
+    F[0], F[1], F[2], F[3] = 2e7, -1e7, 1.5e7 / Z0, 1.5e7 / Z0
+    m.set_fields(F)
+    Fd = m.fields()
+    R0, P0 = m.particles()
+    origin = (inf["origin"][0] - hx, inf["origin"][1] - hy)
+    Ro, Po, _, Rmid = O.push_patch(order, b, dt, Fd[0], Fd[1], Fd[2] + Fd[3], origin, (hx, hy), R0, P0, s2bug=False)
+    m.push(1)
+    R1, P1 = m.particles()
+    J = m.fields()[5][1:-1, 1:-1]
+    Jo = O.deposit(order, 1, (wx0, wy0, m.W, m.H), tuple(b.origin), (hx, hy), dt, R0, Rmid, np.full(n, Q[0]))
+    err = (np.abs((P1 - P0) - (Po - P0)).max() / np.abs(Po - P0).max(), np.abs(R1 - Ro).max() / hx,
+           np.abs(J - Jo).max() / np.abs(Jo).max())
+    print("push %s order %d, %d particles: dP %.2e, R %.2e cells, J %.2e" % (("FP32" if fp32 else "FP64", order, n) + err))
+    tol = (2e-5, 2e-6, 5e-5) if fp32 else (1e-11, 1e-12, 1e-11)
+    assert all(e < t for e, t in zip(err, tol)), err
+
+
 def test_line_fields_vs_oracle(gpu):
     """SaveEMFieldsCommand (SaveEMFields.cpp:34-160) through csrst_line_fields
     after 40 steps into the bend and the copy of the window's E and H that
