@@ -20,10 +20,11 @@
 //   k_push<comp=0>  drift, gather, kick+rotation, drift, S0/S1/S2 deposit of
 //                   Jx (register slots per stencil anchor, wavefront sums
 //                   into an LDS tile, one global atomic per node), drift back
-//   k_heh           H half-step, Ex, H half-step in one row-marching pass
+//   k_sweep         H half-step, Ex, H half-step and, outside the bunch's
+//                   footprint, Ey in one row-marching pass
 //   k_push<comp=1>  same, depositing Jy
-//   k_ey            Ey
-//   k_move          window move decision on the device, ring-offset update
+//   k_late          Ey in the footprint and in the absorbing layers; its last
+//                   workgroup decides the window move (ring-offset update)
 //   k_fresh         clear + geometry for the recycled guard column/row
 // plus a periodic cell sort and the wake sampling.
 #include <hip/hip_runtime.h>
@@ -68,18 +69,30 @@ struct WinState {
     int steps;
     double p0[2];        // reference momentum: particles store P - p0 (re-centred at every sort)
     int sbox[4];         // cell box of the particles at the last sort: min x, min y, -max x, -max y
+    int done;            // workgroups of k_late that have finished
+    // device clock (wall_clock64) at the start of the step's kernels (Tick),
+    // and the sums of this call's steps: push, sweeps, move, sort
+    unsigned long long t[8], sum[4];
 };
+enum Tick { kSort, kPush0, kSweep, kPush1, kLate, kMove, kFreshEnd };
+
+// one thread per kernel notes when it starts; kernels of a stream follow each
+// other, so the differences are the kernels' times with the gaps between them
+__device__ __forceinline__ void tick(WinState *ws, Tick k)
+{
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) ws->t[k] = wall_clock64();
+}
 
 template <class T>
 struct Fields {
     T *ex, *ey, *hz, *jx, *jy;
-    T *ex2, *hz2;        // ping-pong partners of ex and hz (written by k_heh)
+    T *ex2, *ey2, *hz2;  // ping-pong partners of ex, ey and hz (written by k_sweep)
     uint8_t *cls;
     T *cut;              // 5 planes: lam0, lam1, area, lamN0, lamN1
     int W, H, Wp, Hp;    // logical interior size, physical (padded) size
     size_t plane;
     // convolutional PML along x at both window ends (npml columns each):
-    // psi of the x-derivative in the Hz update (ping-pong with k_heh) and in
+    // psi of the x-derivative in the Hz update (ping-pong with k_sweep) and in
     // the Ey update; per logical column: decay b and weight a = b - 1 for
     // the Hz half step (at i + 1/2) and the Ey step (at i)
     int npml;
@@ -165,7 +178,7 @@ __global__ void k_geom_all(Fields<T> f, Geo g, const WinState *ws)
     const int j = blockIdx.y - G;
     if (i > f.W - 1 + G) return;
     const size_t q = (size_t)ringy(j, ws->ry, f.Hp) * f.Wp + ringx(i, ws->rx, f.Wp);
-    f.ex[q] = 0; f.ey[q] = 0; f.hz[q] = 0; f.jx[q] = 0; f.jy[q] = 0; f.ex2[q] = 0; f.hz2[q] = 0;
+    f.ex[q] = 0; f.ey[q] = 0; f.hz[q] = 0; f.jx[q] = 0; f.jy[q] = 0; f.ex2[q] = 0; f.ey2[q] = 0; f.hz2[q] = 0;
     if (f.npml) { f.psih[q] = 0; f.psih2[q] = 0; f.psie[q] = 0; }
     cell_geometry(g, f, ws->wx0 + i, ws->wy0 + j, q);
 }
@@ -594,6 +607,7 @@ constexpr int few_particles(int order)
 template <class T, int ORDER, int COMP, bool MISSCOOP, int PPT>
 __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3))) k_push(Parts<T> p, Fields<T> f, Geo g, PushConst<T> c, WinState *ws)
 {
+    tick(ws, COMP == 0 ? kPush0 : kPush1);
     __shared__ T acc[kTH * kTW];
     __shared__ int pbox[4];          // particle cell box of the chunk (min x, min y, -max x, -max y)
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1009,11 +1023,17 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
 // ---------------------------------------------------------------------------
 // Field sweeps.  Thread = column, marching over a strip of rows.
 //
-// k_heh: H half step, Ex, H half step (TETMSolver.hh:142-206 without the
+// k_sweep: H half step, Ex, H half step (TETMSolver.hh:142-206 without the
 // exchanges, with the conformal cell updates of TETMSolver.cpp:87-115 in
 // place of the bulk update at cut cells).  For row j it computes H1(j)
 // (needs E(j+1) old), Ex(j) (needs H1(j), H1(j-1)), then H2(j-1) (needs
-// Ex(j), Ex(j-1) new).  Ey is read-only in this kernel.
+// Ex(j), Ex(j-1) new), then Ey(j-1) (TETMSolver.hh:241-249, conformal
+// TETMSolver.cpp:117-127; needs H2 of this column and of the one before).  The
+// second push comes between H2 and Ey, but it reads Ey, and deposits Jy, in
+// the bunch's footprint only: there Ey is copied and k_late advances it after
+// the push.  Ex, Ey and Hz go to their partner buffers, since neighbouring
+// columns and strips still read the old values: 25 B per cell in FP32 (49 in
+// FP64) where a sweep for Hz and Ex and another for Ey moved 34 (66).
 template <class T>
 struct SweepConst {
     T sx, sy;            // 0.5 etax / Z0, 0.5 etay / Z0 (bulk H)
@@ -1024,12 +1044,26 @@ struct SweepConst {
     T ihx, ihy;          // 1/hx, 1/hy
 };
 
-// Rows per workgroup of the sweeps.  Short strips give many workgroups to
-// hide HBM latency, which outweighs k_heh's re-read of the rows above and
-// below its strip: at c3 the two sweeps took 1.01 ms per step with 32-row
-// strips, 0.91 ms with 8 and 0.89 ms with 4 (c2: 0.198, 0.160 ms with 4).
-// k_ey loads its rows in one group of four.
-constexpr int kStrip = 4;
+// Rows per wave of the sweep.  Short strips give many waves to hide HBM latency,
+// long ones re-read fewer rows above and below.  us per step with 4, 8, 12, 16
+// rows: c3 (FP32, 134M cells) 805, 738, 736, 731; c5 (FP64) 1558, 1493, 1498,
+// 1517; c1 (512 x 256) 15.7, 15.8, 17.3, 19.9.  c3's launch moves its 3.4 GB in
+// 0.72 ms, 4.7 TB/s; the two sweeps that moved 4.6 GB took 0.89 ms.
+constexpr int kStrip = 8;
+constexpr int kPmlStrip = 8;          // rows per wave in the absorbing layers
+constexpr int kCols = 63;             // columns per wave: lane 0 recomputes the column before for its H
+
+// the footprint of the next deposits in logical cells, clamped to the window
+struct Foot {
+    int x0, y0, x1, y1;
+    __device__ __forceinline__ bool has(int i, int j) const { return i >= x0 && i <= x1 && j >= y0 && j <= y1; }
+};
+__device__ __forceinline__ Foot footprint(const WinState *ws, int W, int H)
+{
+    const int *b = ws->jbox[0];            // the same box for both components
+    if (b[0] == INT_MAX) return Foot{0, 0, -1, -1};
+    return Foot{max(b[0] - ws->wx0, 0), max(b[1] - ws->wy0, 0), min(-b[2] - ws->wx0, W - 1), min(-b[3] - ws->wy0, H - 1)};
+}
 
 template <class T>
 __device__ __forceinline__ T h_update(const Fields<T> &f, size_t q, uint8_t cls, T h, T ey, T eyp, T ex, T exn,
@@ -1056,32 +1090,40 @@ __device__ __forceinline__ T ex_update(const Fields<T> &f, size_t q, uint8_t cls
     return ex;
 }
 
-// Row march for one column i over the strip [j0, j1]: H1 for rows
-// j0-1 .. j1+1, Ex for rows j0 .. j1+1, H2 for rows j0 .. j1; only H2 and Ex
-// of the strip rows are stored, into the partner buffers (ex2, hz2), so the
-// halo rows other strips read are never overwritten during the pass.  Guard
-// rows (-1, H) are never updated.
-// Columns: PML = false sweeps the ncol columns from cbase; PML = true the two
-// end layers (t < npml: column t, else column W - 2 npml + t).
-template <class T, bool PML, int STRIP>
-__global__ void __launch_bounds__(kB) k_heh(Fields<T> f, SweepConst<T> c, const WinState *ws, int jbase, int cbase,
-                                            int ncol)
+// Ey at a cell: d the x difference of H (psi included), jv the current
+template <class T>
+__device__ __forceinline__ T ey_update(const Fields<T> &f, size_t q, uint8_t cls, T ey, T d, T jv, const SweepConst<T> &c)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ncol) return;
-    const int i = PML ? (t < f.npml ? t : f.W - 2 * f.npml + t) : cbase + t;   // logical column
+    if (cls == 1) return ey - (c.sey * d + c.dteps * jv);
+    if (cls == 2 && f.cut[f.plane + q] > T(pm::kSpaceEps) && f.cut[2 * f.plane + q] >= T(pm::kMinArea))
+        return ey + c.ce * (-d * c.ihx - jv);
+    return ey;
+}
+
+__device__ __forceinline__ float from_prev_lane(float v) { return dpp_f<0x138, 0xf>(v); }    // wave_shr:1
+__device__ __forceinline__ double from_prev_lane(double v) { return dpp_d<0x138, 0xf>(v); }
+
+// Row march for one column i over the strip [j0, j1]: H1 for rows
+// j0-1 .. j1+1, Ex for rows j0 .. j1+1, H2 for rows j0 .. j1; only Ey, H2 and Ex
+// of the strip rows are stored, into the partner buffers (ey2, ex2, hz2), so the
+// halo rows other strips read are never overwritten during the pass.  Guard
+// rows (-1, H) and columns (-1, W) are never updated; their Ey is carried over.
+// store: this lane's column is its own (not a halo, not past the end).  eyLo:
+// the first column whose Ey is advanced here, outside the footprint (PML =
+// false, called by whole waves whose lanes hold consecutive columns).
+template <class T, bool PML>
+__device__ __forceinline__ void march(const Fields<T> &f, const SweepConst<T> &c, const WinState *ws, int i, int j0, int j1,
+                                      bool store, int eyLo)
+{
     const int rx = ws->rx, ry = ws->ry;
-    const int j0 = jbase + blockIdx.y * STRIP;
-    if (j0 > f.H - 1) return;
-    const int j1 = min(j0 + STRIP - 1, f.H - 1);
     const int px = ringx(i, rx, f.Wp), pxp = ringx(i + 1, rx, f.Wp);
-    const int jlo0 = ws->jbox[0][0] - ws->wx0, jlo1 = ws->jbox[0][1] - ws->wy0;
-    const int jhi0 = -ws->jbox[0][2] - ws->wx0, jhi1 = -ws->jbox[0][3] - ws->wy0;
-    const bool colInJ = i >= jlo0 && i <= jhi0;
+    const Foot fp = footprint(ws, f.W, f.H);
+    const bool colInJ = i >= fp.x0 && i <= fp.x1;
+    const bool guard = i < 0 || i >= f.W;
     auto row = [&](int j) { return (size_t)ringy(j, ry, f.Hp) * f.Wp; };
     // PML column: Hz's x term (eyp - ey) becomes (eyp - ey) + psi with
     // psi <- b psi + a (eyp - ey)
-    const bool inPml = PML && (i < f.npml || i >= f.W - f.npml);
+    const bool inPml = PML && !guard && (i < f.npml || i >= f.W - f.npml);
     const T bh = inPml ? f.pml[i] : T(0), ah = inPml ? f.pml[f.W + i] : T(0);
     // x difference of the Hz update: Ey(i+1) - Ey(i) in bulk cells, the
     // edge-length weighted n1 Ey(i+1) - l1 Ey(i) in cut cells
@@ -1120,6 +1162,7 @@ __global__ void __launch_bounds__(kB) k_heh(Fields<T> f, SweepConst<T> c, const 
                       f.ex[row(j0) + px], inPml ? f.psih[rb + px] : T(0), psi1, true);
         } else {
             h1p = hold;
+            if (store) f.ey2[rb + px] = f.ey[rb + px];
         }
     }
     T psi1p = 0;
@@ -1127,7 +1170,7 @@ __global__ void __launch_bounds__(kB) k_heh(Fields<T> f, SweepConst<T> c, const 
     T exnp = 0, eyp_prev = 0, ey_prev = 0, h1pp = 0;
     uint8_t clp = 0;
     size_t qprev = 0;
-    // the march's loads run one row ahead of its arithmetic
+    // the march's loads run two rows ahead of its arithmetic
     struct RowIn {
         T ey, eyp, hz, jv, psi, exnext;
         uint8_t cl;
@@ -1139,13 +1182,14 @@ __global__ void __launch_bounds__(kB) k_heh(Fields<T> f, SweepConst<T> c, const 
         r.hz = f.hz[q];
         r.cl = f.cls[q];
         r.exnext = f.ex[row(j + 1) + px];
-        r.jv = (colInJ && j >= jlo1 && j <= jhi1 && j <= f.H - 1) ? f.jx[q] : T(0);
+        r.jv = (colInJ && j >= fp.y0 && j <= fp.y1) ? f.jx[q] : T(0);
         r.psi = inPml ? f.psih[q] : T(0);
     };
-    RowIn cur, nxt;
+    RowIn cur, nxt, nx2;
     fetch(j0, cur);
+    fetch(j0 + 1, nxt);
     for (int j = j0; j <= j1 + 1; ++j) {
-        if (j + 1 <= j1 + 1) fetch(j + 1, nxt);
+        if (j + 2 <= j1 + 1) fetch(j + 2, nx2);
         const size_t q = row(j) + px;
         const T exo_next = cur.exnext;
         const T ey = cur.ey, eyp = cur.eyp;
@@ -1157,13 +1201,28 @@ __global__ void __launch_bounds__(kB) k_heh(Fields<T> f, SweepConst<T> c, const 
         } else {
             h1 = cur.hz;
             exn = exo;
+            if (store) f.ey2[q] = ey;
         }
         if (j > j0) {
             // H2(j-1) from H1(j-1), Ex new at j-1 and j
             T psi2 = 0;
-            f.hz2[qprev] = hup(qprev, clp, h1pp, ey_prev, eyp_prev, exnp, exn, psi1p, psi2, false);
-            if (inPml) f.psih2[qprev] = psi2;
-            f.ex2[qprev] = exnp;
+            T h2 = hup(qprev, clp, h1pp, ey_prev, eyp_prev, exnp, exn, psi1p, psi2, false);
+            T eyn = ey_prev;
+            if (!PML) {
+                // a guard column keeps what its buffer holds
+                if (i < 0) h2 = f.hz2[qprev];
+                const T left = from_prev_lane(h2);
+                if (i >= eyLo && !(colInJ && j - 1 >= fp.y0 && j - 1 <= fp.y1))
+                    eyn = ey_update(f, qprev, clp, ey_prev, h2 - left, T(0), c);
+            }
+            if (store) {
+                f.ey2[qprev] = guard ? ey_prev : eyn;
+                if (!guard) {
+                    f.hz2[qprev] = h2;
+                    f.ex2[qprev] = exnp;
+                    if (inPml) f.psih2[qprev] = psi2;
+                }
+            }
         }
         psi1p = psi1;
         h1pp = h1;
@@ -1172,87 +1231,139 @@ __global__ void __launch_bounds__(kB) k_heh(Fields<T> f, SweepConst<T> c, const 
         exo = exo_next;
         ey_prev = ey; eyp_prev = eyp; clp = cl; qprev = q;
         cur = nxt;
+        nxt = nx2;
     }
 }
 
-// Ey (TETMSolver.hh:241-249, conformal TETMSolver.cpp:117-127); clears Jy in
-// its footprint after use and Jx in the Jx footprint, leaving both current
-// planes zero for the next deposits.
-template <class T, bool PML, int STRIP>
-__global__ void __launch_bounds__(kB) k_ey(Fields<T> f, SweepConst<T> c, const WinState *ws, int cbase, int ncol)
+// The sweep of the whole window: the absorbing layers' waves first (2 npml
+// columns and the two guard columns, kPmlStrip rows each), then the interior's
+// (columns npml .. W - npml - 1, kCols per wave; without absorbing layers the
+// guard columns are here).  One launch, so the few layer waves, whose rows take
+// longest, run beside the rest.
+template <class T>
+__global__ void __launch_bounds__(kB) k_sweep(Fields<T> f, SweepConst<T> c, WinState *ws, int pmlBlocks, int gx)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ncol) return;
-    const int i = PML ? (t < f.npml ? t : f.W - 2 * f.npml + t) : cbase + t;
-    const int rx = ws->rx, ry = ws->ry;
-    const int px = ringx(i, rx, f.Wp), pxm = ringx(i - 1, rx, f.Wp);
-    const int jlo0 = ws->jbox[1][0] - ws->wx0, jlo1 = ws->jbox[1][1] - ws->wy0;
-    const int jhi0 = -ws->jbox[1][2] - ws->wx0, jhi1 = -ws->jbox[1][3] - ws->wy0;
-    const bool colInJ = i >= jlo0 && i <= jhi0;
-    const int xlo0 = ws->jbox[0][0] - ws->wx0, xlo1 = ws->jbox[0][1] - ws->wy0;
-    const int xhi0 = -ws->jbox[0][2] - ws->wx0, xhi1 = -ws->jbox[0][3] - ws->wy0;
-    const bool colInJx = i >= xlo0 && i <= xhi0;
-    const bool inPml = PML && (i < f.npml || i >= f.W - f.npml);
-    const T be = inPml ? f.pml[2 * f.W + i] : T(0), ae = inPml ? f.pml[3 * f.W + i] : T(0);
-    const int j0 = blockIdx.y * STRIP, j1 = min(j0 + STRIP - 1, f.H - 1);
-    // rows are independent: each group of four issues all its loads before
-    // any arithmetic or store
-    constexpr int G4 = 4;
-    for (int jb = j0; jb <= j1; jb += G4) {
-        size_t qv[G4];
-        uint8_t clv[G4];
-        T dv[G4], eyv[G4], jvv[G4], psv[G4];
+    tick(ws, kSweep);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int np = f.npml;
+    if ((int)blockIdx.x < pmlBlocks) {
+        const int strips = (f.H + kPmlStrip - 1) / kPmlStrip;
+        const int w = blockIdx.x * (kB / 64) + wave;
+        const int t = (w / strips) * 64 + lane, j0 = (w % strips) * kPmlStrip;
+        if (t >= 2 * np + 2) return;
+        const int i = t < np ? t : t < 2 * np ? f.W - 2 * np + t : t == 2 * np ? -1 : f.W;
+        march<T, true>(f, c, ws, i, j0, min(j0 + kPmlStrip - 1, f.H - 1), true, 0);
+        return;
+    }
+    // Consecutive workgroups run on the 8 XCDs in turn: each XCD takes a
+    // contiguous part of the window, so that the rows a strip shares with the
+    // ones above and below come from its own L2 (pmlBlocks is a multiple of 8).
+    const int n = gridDim.x - pmlBlocks, b = blockIdx.x - pmlBlocks;
+    const int L = b < (n & ~7) ? (b & 7) * (n >> 3) + (b >> 3) : b;
+    const int first = np ? np : -1, last = np ? f.W - np - 1 : f.W;   // columns to store
+    const int j0 = (L / gx) * kStrip, w = (L % gx) * (kB / 64) + wave;
+    // lane 0 is the column before; the first wave's lane 0 is the guard column
+    // (its own) or an absorbing column, whose H this pass does not compute: Ey
+    // of the column after that is left to k_late
+    const int c0 = first + (np ? 0 : 1) + kCols * w, i = c0 - 1 + lane;
+    if (c0 > last) return;                                            // uniform
+    const bool store = i >= first && i <= last && (lane > 0 || i < 0);
+    march<T, false>(f, c, ws, min(i, f.W), j0, min(j0 + kStrip - 1, f.H - 1), store, np ? np + 1 : 0);
+}
+
+// Ey where the sweep left it: in the footprint, in the absorbing layers, and in
+// the column after the leading one.  Clears Jx and Jy in the footprint, leaving
+// both current planes zero for the next deposits.  Work units of 64 columns x 4
+// rows (64 rows of the single column), all loads of a unit before its stores,
+// walked by at most kLateBlocks workgroups: the last of them to finish ends the
+// step (the move for lead >= 0, and the step's times), and the count of finished
+// workgroups is one address that all XCDs update (with 3000 workgroups and a
+// device fence in each, this kernel took 156 us at 16384 x 8192; 18 us now).
+constexpr int kLateBlocks = 256;
+__device__ void window_move(WinState *ws, int t, int W, int H, int Wp, int Hp, int lead);
+__device__ void end_of_step(WinState *ws, bool pushed, bool sorted);
+
+template <class T>
+__global__ void __launch_bounds__(kB) k_late(Fields<T> f, SweepConst<T> c, WinState *ws, int lead, bool pushed, bool sorted)
+{
+    tick(ws, kLate);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int rx = ws->rx, ry = ws->ry, np = f.npml;
+    const Foot fp = footprint(ws, f.W, f.H);
+    constexpr int R = 4;
+    // rows j .. j + R - 1 (to jEnd) of column i; pml: in an absorbing layer
+    auto cells = [&](int i, int j, int jEnd, bool pml) {
+        const int px = ringx(i, rx, f.Wp), pxm = ringx(i - 1, rx, f.Wp);
+        const T be = pml ? f.pml[2 * f.W + i] : T(0), ae = pml ? f.pml[3 * f.W + i] : T(0);
+        size_t q[R];
+        T d[R], ey[R], jv[R], psi[R];
+        uint8_t cl[R];
 #pragma unroll
-        for (int u = 0; u < G4; ++u) {
-            const int j = min(jb + u, j1);
-            const size_t rb = (size_t)ringy(j, ry, f.Hp) * f.Wp;
-            const size_t q = rb + px;
-            qv[u] = q;
-            clv[u] = f.cls[q];
-            dv[u] = f.hz[q] - f.hz[rb + pxm];
-            eyv[u] = f.ey[q];
-            jvv[u] = (colInJ && j >= jlo1 && j <= jhi1) ? f.jy[q] : T(0);
-            psv[u] = (PML && inPml) ? f.psie[q] : T(0);
+        for (int u = 0; u < R; ++u) {
+            const size_t rb = (size_t)ringy(min(j + u, jEnd), ry, f.Hp) * f.Wp;
+            q[u] = rb + px;
+            d[u] = f.hz[q[u]] - f.hz[rb + pxm];
+            cl[u] = f.cls[q[u]];
+            ey[u] = f.ey[q[u]];
+            jv[u] = fp.has(i, j + u) ? f.jy[q[u]] : T(0);
+            psi[u] = pml ? f.psie[q[u]] : T(0);
         }
 #pragma unroll
-        for (int u = 0; u < G4; ++u) {
-            const int j = jb + u;
-            if (j > j1) break;
-            const size_t q = qv[u];
-            const uint8_t cl = clv[u];
-            const T d = dv[u], jv = jvv[u];
-            if (colInJ && j >= jlo1 && j <= jhi1) f.jy[q] = 0;
-            if (colInJx && j >= xlo1 && j <= xhi1) f.jx[q] = 0;
-            if (cl == 1) {
-                T dd = d;
-                if (PML && inPml) {
-                    const T psi = be * psv[u] + ae * d;
-                    f.psie[q] = psi;
-                    dd = d + psi;
-                }
-                f.ey[q] = eyv[u] - (c.sey * dd + c.dteps * jv);
-            } else if (cl == 2 && f.cut[f.plane + q] > T(pm::kSpaceEps) && f.cut[2 * f.plane + q] >= T(pm::kMinArea)) {
-                T dd = d;
-                if (PML && inPml) {
-                    const T psi = be * psv[u] + ae * d;
-                    f.psie[q] = psi;
-                    dd = d + psi;
-                }
-                f.ey[q] = eyv[u] + c.ce * (-dd * c.ihx - jv);
+        for (int u = 0; u < R; ++u) {
+            if (j + u > jEnd) break;
+            const size_t k = q[u];
+            if (fp.has(i, j + u)) {
+                f.jy[k] = 0;
+                f.jx[k] = 0;
             }
+            T dd = d[u];
+            if (pml && (cl[u] == 1 || (cl[u] == 2 && f.cut[f.plane + k] > T(pm::kSpaceEps) &&
+                                       f.cut[2 * f.plane + k] >= T(pm::kMinArea)))) {
+                const T ps = be * psi[u] + ae * dd;
+                f.psie[k] = ps;
+                dd = dd + ps;
+            }
+            f.ey[k] = ey_update(f, k, cl[u], ey[u], dd, jv[u], c);
+        }
+    };
+    // units: the footprint's interior columns, the layers' 2 np columns, column np
+    const int x0 = max(fp.x0, np ? np + 1 : 0), x1 = min(fp.x1, f.W - np - 1);
+    const int bw = max((x1 - x0 + 64) / 64, 0), uBox = bw * max((fp.y1 - fp.y0 + R) / R, 0);
+    const int rows = (f.H + R - 1) / R, uPml = (2 * np + 63) / 64 * rows, uCol = np ? (f.H + 63) / 64 : 0;
+    for (int u = blockIdx.x * (kB / 64) + wave; u < uBox + uPml + uCol; u += gridDim.x * (kB / 64)) {
+        if (u < uBox) {
+            const int i = x0 + u % bw * 64 + lane;
+            if (i <= x1) cells(i, fp.y0 + u / bw * R, fp.y1, false);
+        } else if (u < uBox + uPml) {
+            const int v = u - uBox, t = v / rows * 64 + lane;
+            if (t < 2 * np) cells(t < np ? t : f.W - 2 * np + t, v % rows * R, f.H - 1, true);
+        } else {
+            const int j = (u - uBox - uPml) * 64 + lane;
+            if (j < f.H) cells(np, j, j, false);
         }
     }
+    __shared__ bool last;
+    __syncthreads();
+    // relaxed: the last workgroup uses nothing that the others wrote, they only
+    // have to be done with the window state
+    if (threadIdx.x == 0) last = atomicAdd(&ws->done, 1) == (int)gridDim.x - 1;
+    __syncthreads();
+    if (!last || wave) return;
+    if (lane == 0) {
+        ws->done = 0;
+        end_of_step(ws, pushed, sorted);
+    }
+    if (lead >= 0) window_move(ws, lane, f.W, f.H, f.Wp, f.Hp, lead);
 }
 
 // ---------------------------------------------------------------------------
 // window move decision: keep the bunch's leading edge `lead` cells from the
 // window front and its centre near the window centre in y (at most one cell
 // per axis per step, as moveMesh, main.cpp:562-652).
-// one wavefront: reduce and clear the kBBSlots particle-box slots, then
-// lane 0 decides the move
-__global__ void k_move(WinState *ws, int W, int H, int Wp, int Hp, int lead)
+// Called by one wavefront (t: the lane): reduces and clears the kBBSlots
+// particle-box slots, then lane 0 decides the move.
+__device__ void window_move(WinState *ws, int t, int W, int H, int Wp, int Hp, int lead)
 {
-    const int t = threadIdx.x;
     int b[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -1261,6 +1372,8 @@ __global__ void k_move(WinState *ws, int W, int H, int Wp, int Hp, int lead)
         b[c] = hu::wave_min(b[c]);
     }
     if (t != 0) return;
+    ws->t[kMove] = wall_clock64();
+    ws->t[kFreshEnd] = 0;
     for (int c = 0; c < 4; ++c) ws->bb[c] = b[c];
     const int bmaxx = -ws->bb[2] - ws->wx0;
     const int bminy = ws->bb[1] - ws->wy0, bmaxy = -ws->bb[3] - ws->wy0;
@@ -1280,10 +1393,31 @@ __global__ void k_move(WinState *ws, int W, int H, int Wp, int Hp, int lead)
     ws->bb[0] = INT_MAX; ws->bb[1] = INT_MAX; ws->bb[2] = INT_MAX; ws->bb[3] = INT_MAX;
     ws->steps += 1;
 }
+__global__ void k_move(WinState *ws, int W, int H, int Wp, int Hp, int lead) { window_move(ws, threadIdx.x, W, H, Wp, Hp, lead); }
+
+// the step's times into the call's sums (the move of this step ends later: the
+// next step adds it, or the host after the last)
+__device__ void end_of_step(WinState *ws, bool pushed, bool sorted)
+{
+    const unsigned long long now = wall_clock64();
+    unsigned long long *t = ws->t;
+    if (t[kFreshEnd] > t[kMove]) ws->sum[2] += t[kFreshEnd] - t[kMove];
+    t[kFreshEnd] = 0;
+    if (pushed) ws->sum[0] += (t[kSweep] - t[kPush0]) + (t[kLate] - t[kPush1]);
+    ws->sum[1] += (pushed ? t[kPush1] - t[kSweep] : t[kLate] - t[kSweep]) + (now - t[kLate]);
+    if (sorted) ws->sum[3] += t[kPush0] - t[kSort];
+}
+
+// the times of a csrst_mw_step call start at zero
+__global__ void k_clear_times(WinState *ws)
+{
+    for (int k = 0; k < 4; ++k) ws->sum[k] = 0;
+    for (int k = 0; k < 8; ++k) ws->t[k] = 0;
+}
 
 // clear + geometry of the recycled guard column (mi = 1) / row (mj = +-1)
 template <class T>
-__global__ void k_fresh(Fields<T> f, Geo g, const WinState *ws)
+__device__ __forceinline__ void fresh_cell(const Fields<T> &f, const Geo &g, const WinState *ws)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int mi = ws->mi, mj = ws->mj;
@@ -1305,9 +1439,16 @@ __global__ void k_fresh(Fields<T> f, Geo g, const WinState *ws)
         return;
     }
     const size_t q = (size_t)ringy(j, ws->ry, f.Hp) * f.Wp + ringx(i, ws->rx, f.Wp);
-    f.ex[q] = 0; f.ey[q] = 0; f.hz[q] = 0; f.jx[q] = 0; f.jy[q] = 0; f.ex2[q] = 0; f.hz2[q] = 0;
+    f.ex[q] = 0; f.ey[q] = 0; f.hz[q] = 0; f.jx[q] = 0; f.jy[q] = 0; f.ex2[q] = 0; f.ey2[q] = 0; f.hz2[q] = 0;
     if (f.npml) { f.psih[q] = 0; f.psih2[q] = 0; f.psie[q] = 0; }
     cell_geometry(g, f, ws->wx0 + i, ws->wy0 + j, q);
+}
+template <class T>
+__global__ void __launch_bounds__(kB) k_fresh(Fields<T> f, Geo g, WinState *ws)
+{
+    fresh_cell(f, g, ws);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(&ws->t[kFreshEnd], (unsigned long long)wall_clock64());
 }
 
 // ---------------------------------------------------------------------------
@@ -1454,8 +1595,9 @@ __global__ void k_sort_keys(Parts<T> p, const WinState *ws, unsigned *keys, int 
 // Cell box of the particles (min x, min y, -max x, -max y) for the sort
 // keys: per-block minima, then one block reduces them into ws->sbox.
 template <class T>
-__global__ void __launch_bounds__(kB) k_box_partial(Parts<T> p, int *partial)
+__global__ void __launch_bounds__(kB) k_box_partial(Parts<T> p, int *partial, WinState *ws)
 {
+    tick(ws, kSort);
     __shared__ int sh[kB / 64][4];
     int b[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};
     for (int k = blockIdx.x * kB + threadIdx.x; k < p.n; k += gridDim.x * kB) {
@@ -1668,6 +1810,9 @@ __global__ void k_state_init(WinState *ws, int wx0, int wy0)
         for (int k = 0; k < 4; ++k) ws->jbox[c][k] = INT_MAX;
     ws->err = 0;
     ws->steps = 0;
+    ws->done = 0;
+    for (int k = 0; k < 8; ++k) ws->t[k] = 0;
+    for (int k = 0; k < 4; ++k) ws->sum[k] = 0;
 }
 
 __global__ void k_set_p0(WinState *ws, double p0x, double p0y)
@@ -1725,11 +1870,11 @@ struct csrst_mw {
     int nsWake = 0;
     int steps = 0;
     int lead = 32;
-    hipEvent_t ev[16];          // two slots of a step's eight timing events (csrst_mw_step alternates)
+    hipEvent_t ev[4];           // around the two pushes of a step that tries a push form
     double lastMs[5] = {0, 0, 0, 0, 0};
     bool ready = false;
 
-    int cur = 0;   // which of the Ex/Hz (and PML psi) ping-pong buffers is current
+    int cur = 0;   // which of the Ex/Ey/Hz (and PML psi) ping-pong buffers is current
     int npml = 0;  // PML columns at each window end
     // the push sends slot misses through the wavefront (MISSCOOP).  Chosen by
     // timing: every kRetune steps one step runs each form and the faster stays
@@ -1745,9 +1890,11 @@ struct csrst_mw {
         mw::Fields<T> f;
         T *b = reinterpret_cast<T *>(fieldsBuf.p);
         T *exa = b, *exb = b + 5 * plane, *hza = b + 2 * plane, *hzb = b + 6 * plane;
+        T *eya = b + plane, *eyb = b + 12 * plane;
         f.ex = cur ? exb : exa; f.ex2 = cur ? exa : exb;
+        f.ey = cur ? eyb : eya; f.ey2 = cur ? eya : eyb;
         f.hz = cur ? hzb : hza; f.hz2 = cur ? hza : hzb;
-        f.ey = b + plane; f.jx = b + 3 * plane; f.jy = b + 4 * plane;
+        f.jx = b + 3 * plane; f.jy = b + 4 * plane;
         f.cut = b + 7 * plane;
         f.cls = cls.p;
         f.W = W; f.H = H; f.Wp = Wp; f.Hp = Hp; f.plane = plane;
@@ -1852,7 +1999,7 @@ void sort_particles(csrst_mw *m)
 {
     const int nb = (m->n + mw::kB - 1) / mw::kB;
     int *boxPart = reinterpret_cast<int *>(m->partial.p);   // kRedBlocks x 4 ints
-    mw::k_box_partial<T><<<mw::kRedBlocks, mw::kB, 0, m->s>>>(m->parts<T>(m->partBuf), boxPart);
+    mw::k_box_partial<T><<<mw::kRedBlocks, mw::kB, 0, m->s>>>(m->parts<T>(m->partBuf), boxPart, m->ws.p);
     mw::k_box_final<<<1, mw::kB, 0, m->s>>>(boxPart, mw::kRedBlocks, m->ws.p);
     mw::k_sort_keys<T><<<nb, mw::kB, 0, m->s>>>(m->parts<T>(m->partBuf), m->ws.p, m->keys.p, m->idx.p);
     HU_LAUNCH_CHECK();
@@ -1878,48 +2025,48 @@ void wake(csrst_mw *m)
     HU_LAUNCH_CHECK();
 }
 
+// timed: the step's pushes between events (the comparison of the push forms)
 template <class T>
-void one_step(csrst_mw *m, bool timed, int slot)
+void one_step(csrst_mw *m, bool timed)
 {
-    hipEvent_t *ev = m->ev + 8 * slot;
+    hipEvent_t *ev = m->ev;
     mw::SweepConst<T> sc;
     sweep_consts(m, sc);
     const mw::Fields<T> f = m->fields<T>();
-    // interior columns without PML terms; the two PML layers in a launch of their own
-    const int np = m->npml, nin = m->W - 2 * np;
-    const dim3 gs((nin + mw::kB - 1) / mw::kB, (m->H + mw::kStrip - 1) / mw::kStrip);
-    // the PML columns are few: one wavefront of columns per workgroup and
-    // short strips, so that the launch still spreads over the chip
-    constexpr int kPmlStrip = 8;
-    const dim3 gp((2 * np + 63) / 64, (m->H + kPmlStrip - 1) / kPmlStrip);
-    if (m->n > 0 && m->p.sortEvery > 0 && m->steps % m->p.sortEvery == 0) {
-        if (timed) HU_CHECK(hipEventRecord(ev[6], m->s));
-        sort_particles<T>(m);
-        if (timed) HU_CHECK(hipEventRecord(ev[7], m->s));
-    }
+    const int np = m->npml, W = m->W, H = m->H;
+    constexpr int kW = mw::kB / 64;
+    auto waves = [](int n, int per) { return (n + per - 1) / per; };
+    // the sweep: interior columns (and, without layers, the guard columns) by
+    // strips; the layers' waves in extra rows of the grid
+    const int cols = np ? W - 2 * np : W + 1, gx = waves(waves(cols, mw::kCols), kW);
+    const int pmlBlocks = np ? (waves(waves(2 * np + 2, 64) * waves(H, mw::kPmlStrip), kW) + 7) & ~7 : 0;
+    const int gs = pmlBlocks + gx * waves(H, mw::kStrip);
+    const int nLate = std::min(mw::kLateBlocks, (int)(((size_t)W * H + 2047) / 2048));
+    const bool sorted = m->n > 0 && m->p.sortEvery > 0 && m->steps % m->p.sortEvery == 0;
+    const bool sample = m->n > 0 && m->p.statModulus > 0 && m->steps % m->p.statModulus == m->p.statModulus - 1;
+    if (sorted) sort_particles<T>(m);
     if (timed) HU_CHECK(hipEventRecord(ev[0], m->s));
     if (m->n > 0) push_dispatch<T, 0>(m);
     if (timed) HU_CHECK(hipEventRecord(ev[1], m->s));
-    hipLaunchKernelGGL((mw::k_heh<T, false, mw::kStrip>), gs, dim3(mw::kB), 0, m->s, f, sc, m->ws.p, 0, np, nin);
-    if (np) hipLaunchKernelGGL((mw::k_heh<T, true, kPmlStrip>), gp, dim3(64), 0, m->s, f, sc, m->ws.p, 0, 0, 2 * np);
+    mw::k_sweep<T><<<gs, mw::kB, 0, m->s>>>(f, sc, m->ws.p, pmlBlocks, gx);
     HU_LAUNCH_CHECK();
     m->cur ^= 1;
     const mw::Fields<T> f2 = m->fields<T>();
     if (timed) HU_CHECK(hipEventRecord(ev[2], m->s));
     if (m->n > 0) push_dispatch<T, 1>(m);
     if (timed) HU_CHECK(hipEventRecord(ev[3], m->s));
-    hipLaunchKernelGGL((mw::k_ey<T, false, mw::kStrip>), gs, dim3(mw::kB), 0, m->s, f2, sc, m->ws.p, np, nin);
-    if (np) hipLaunchKernelGGL((mw::k_ey<T, true, kPmlStrip>), gp, dim3(64), 0, m->s, f2, sc, m->ws.p, 0, 2 * np);
+    // the wake is sampled before the window moves
+    mw::k_late<T><<<nLate, mw::kB, 0, m->s>>>(f2, sc, m->ws.p, m->n > 0 && !sample ? m->lead : -1, m->n > 0, sorted);
     HU_LAUNCH_CHECK();
-    if (m->n > 0 && m->p.statModulus > 0 && m->steps % m->p.statModulus == m->p.statModulus - 1) wake<T>(m);
-    if (timed) HU_CHECK(hipEventRecord(ev[4], m->s));
+    if (sample) {
+        wake<T>(m);
+        mw::k_move<<<1, 64, 0, m->s>>>(m->ws.p, W, H, m->Wp, m->Hp, m->lead);
+    }
     if (m->n > 0) {
-        mw::k_move<<<1, 64, 0, m->s>>>(m->ws.p, m->W, m->H, m->Wp, m->Hp, m->lead);
-        const int nf = 2 * (m->H + 2 * mw::G) + m->W + 2 * mw::G;
-        hipLaunchKernelGGL((mw::k_fresh<T>), dim3((nf + mw::kB - 1) / mw::kB), dim3(mw::kB), 0, m->s, f2, m->geo, m->ws.p);
+        const int nf = 2 * (H + 2 * mw::G) + W + 2 * mw::G;
+        mw::k_fresh<T><<<waves(nf, mw::kB), mw::kB, 0, m->s>>>(f2, m->geo, m->ws.p);
         HU_LAUNCH_CHECK();
     }
-    if (timed) HU_CHECK(hipEventRecord(ev[5], m->s));
     ++m->steps;
 }
 
@@ -1928,13 +2075,14 @@ void one_step(csrst_mw *m, bool timed, int slot)
 // the slower form)
 constexpr int kRetune = 200;
 
-void check_state(csrst_mw *m)
+mw::WinState check_state(csrst_mw *m)
 {
     mw::WinState h;
     HU_CHECK(hipMemcpyAsync(&h, m->ws.p, sizeof(h), hipMemcpyDeviceToHost, m->s));
     HU_CHECK(hipStreamSynchronize(m->s));
     if (h.err & 1) throw Error(CSRST_EWINDOW, "particle stencil left the window");
     if (h.err & 2) throw Error(CSRST_EWINDOW, "particle crossed too many cell lines in one push");
+    return h;
 }
 
 }  // namespace
@@ -2061,7 +2209,7 @@ int csrst_mw_create(const csrst_mw_params *p, csrst_mw **out)
         const size_t rs = m->f32 ? 4 : 8;
         // the push gathers address a field plane with 32-bit byte offsets
         if (m->plane * rs > 0xffffffffull) throw Error(CSRST_EINVAL, "window plane exceeds 4 GiB");
-        m->fieldsBuf.alloc(m->plane * 12 * rs);   // ex ey hz jx jy ex' hz' + 5 cut planes
+        m->fieldsBuf.alloc(m->plane * 13 * rs);   // ex ey hz jx jy ex' hz' + 5 cut planes + ey'
         m->fieldsBuf.zero(m->s);
         if (p->pml < 0 || 2 * p->pml > p->W - 8) throw Error(CSRST_EINVAL, "pml must be in [0, (W - 8) / 2]");
         // sort keys: a 16x4-cell tile index over the particles' box (at most
@@ -2230,55 +2378,43 @@ int csrst_mw_step(csrst_mw *m, int nsteps)
 {
     try {
         if (!m || !m->ready) throw Error(CSRST_ESTATE, "csrst_mw_step before csrst_mw_init_bunch");
-        double acc[5] = {0, 0, 0, 0, 0};
-        // Step k records its timing events in slot k % 2, and the host reads
-        // them after it has queued step k + 1, so the GPU never idles while
-        // the host waits.  The comparison of the two slot-miss forms (a
-        // cooperative trial step, then a per-lane one) therefore decides one
-        // step after the per-lane trial ends; that step keeps the per-lane form.
-        int role[2] = {0, 0};              // per slot: 0 none, 1 cooperative trial, 2 per-lane trial
-        bool sorted[2] = {false, false};
-        auto read = [&](int b) {
-            hipEvent_t *e = m->ev + 8 * b;
-            HU_CHECK(hipEventSynchronize(e[5]));
-            float t01, t12, t23, t34, t45, t67 = 0;
-            HU_CHECK(hipEventElapsedTime(&t01, e[0], e[1]));
-            HU_CHECK(hipEventElapsedTime(&t12, e[1], e[2]));
-            HU_CHECK(hipEventElapsedTime(&t23, e[2], e[3]));
-            HU_CHECK(hipEventElapsedTime(&t34, e[3], e[4]));
-            HU_CHECK(hipEventElapsedTime(&t45, e[4], e[5]));
-            if (role[b] == 1) {
-                m->tuneMs = t01 + t23;
-            } else if (role[b] == 2) {
-                m->tilted = m->tuneMs < t01 + t23;
-                m->tunePhase = 0;
-                m->nextTune = m->steps + kRetune;
-            }
-            if (sorted[b]) HU_CHECK(hipEventElapsedTime(&t67, e[6], e[7]));
-            acc[0] += t01 + t23;
-            acc[1] += t12 + t34;
-            acc[2] += t45;
-            acc[3] += t67;
+        // Times come from the device clock, which the step's own kernels note;
+        // events between the kernels cost 55 us of a 120 us step of the
+        // smallest window.  Only a step that tries a push form has them, and
+        // the host waits for it (two steps in kRetune).
+        mw::k_clear_times<<<1, 1, 0, m->s>>>(m->ws.p);
+        auto push_ms = [&]() {
+            HU_CHECK(hipEventSynchronize(m->ev[3]));
+            float a, b;
+            HU_CHECK(hipEventElapsedTime(&a, m->ev[0], m->ev[1]));
+            HU_CHECK(hipEventElapsedTime(&b, m->ev[2], m->ev[3]));
+            return a + b;
         };
+        const bool two = m->n > (m->f32 ? mw::few_particles<float>(m->p.order) : mw::few_particles<double>(m->p.order));
         for (int k = 0; k < nsteps; ++k) {
-            const int b = k & 1;
-            sorted[b] = m->n > 0 && m->p.sortEvery > 0 && m->steps % m->p.sortEvery == 0;
-            role[b] = 0;
-            if (m->n > 0 && m->tunePhase == 0 && m->steps >= m->nextTune) {
+            bool trial = false;
+            if (two && m->tunePhase == 0 && m->steps >= m->nextTune) {
                 m->tunePhase = 1;           // this step runs the cooperative form
-                m->tilted = true;
-                role[b] = 1;
+                m->tilted = trial = true;
             } else if (m->tunePhase == 1) {
                 m->tunePhase = 2;           // and this one the per-lane form
                 m->tilted = false;
-                role[b] = 2;
+                trial = true;
             }
-            if (m->f32) one_step<float>(m, true, b); else one_step<double>(m, true, b);
-            if (k > 0) read(b ^ 1);
+            if (m->f32) one_step<float>(m, trial); else one_step<double>(m, trial);
+            if (trial && m->tunePhase == 1) {
+                m->tuneMs = push_ms();
+            } else if (trial) {
+                m->tilted = m->tuneMs < push_ms();
+                m->tunePhase = 0;
+                m->nextTune = m->steps + kRetune;
+            }
         }
-        if (nsteps > 0) read((nsteps - 1) & 1);
-        for (int k = 0; k < 4; ++k) m->lastMs[k] = nsteps ? acc[k] / nsteps : 0;
-        check_state(m);
+        const mw::WinState h = check_state(m);
+        unsigned long long sum[4];
+        for (int k = 0; k < 4; ++k) sum[k] = h.sum[k];
+        if (h.t[mw::kFreshEnd] > h.t[mw::kMove]) sum[2] += h.t[mw::kFreshEnd] - h.t[mw::kMove];
+        for (int k = 0; k < 4; ++k) m->lastMs[k] = nsteps ? sum[k] * 1e-5 / nsteps : 0;   // the clock ticks every 10 ns
         return CSRST_OK;
     } catch (const std::exception &e) {
         return mw_fail(m, e);
@@ -2344,10 +2480,13 @@ int csrst_mw_upload_fields(csrst_mw *m, const double *in, int count)
         mw::WinState h;
         HU_CHECK(hipMemcpy(&h, m->ws.p, sizeof(h), hipMemcpyDeviceToHost));
         const size_t rs = m->f32 ? 4 : 8;
-        std::vector<unsigned char> raw(7 * m->plane * rs);
-        HU_CHECK(hipMemcpy(raw.data(), m->fieldsBuf.p, raw.size(), hipMemcpyDeviceToHost));
-        const int exPlane = m->cur ? 5 : 0, hzPlane = m->cur ? 6 : 2;
-        const int dst[5] = {exPlane, 1, hzPlane, 3, 4};
+        // planes 0 .. 6, and Ey's partner as plane 7
+        std::vector<unsigned char> raw(8 * m->plane * rs);
+        const size_t head = 7 * m->plane * rs, one = m->plane * rs, eyb = 12 * m->plane * rs;
+        HU_CHECK(hipMemcpy(raw.data(), m->fieldsBuf.p, head, hipMemcpyDeviceToHost));
+        HU_CHECK(hipMemcpy(raw.data() + head, m->fieldsBuf.p + eyb, one, hipMemcpyDeviceToHost));
+        const int exPlane = m->cur ? 5 : 0, eyPlane = m->cur ? 7 : 1, hzPlane = m->cur ? 6 : 2;
+        const int dst[5] = {exPlane, eyPlane, hzPlane, 3, 4};
         for (int pl = 0; pl < 5; ++pl)
             for (int j = -mw::G; j < m->H + mw::G; ++j)
                 for (int i = -mw::G; i < m->W + mw::G; ++i) {
@@ -2363,7 +2502,8 @@ int csrst_mw_upload_fields(csrst_mw *m, const double *in, int count)
                     if (m->f32) { float fv = (float)v; memcpy(d, &fv, 4); }
                     else memcpy(d, &v, 8);
                 }
-        HU_CHECK(hipMemcpy(m->fieldsBuf.p, raw.data(), raw.size(), hipMemcpyHostToDevice));
+        HU_CHECK(hipMemcpy(m->fieldsBuf.p, raw.data(), head, hipMemcpyHostToDevice));
+        HU_CHECK(hipMemcpy(m->fieldsBuf.p + eyb, raw.data() + head, one, hipMemcpyHostToDevice));
         return CSRST_OK;
     } catch (const std::exception &e) {
         return mw_fail(m, e);
@@ -2389,12 +2529,15 @@ int csrst_mw_download_fields(csrst_mw *m, double *out, int cap, int *count)
         mw::WinState h;
         HU_CHECK(hipMemcpy(&h, m->ws.p, sizeof(h), hipMemcpyDeviceToHost));
         const size_t rs = m->f32 ? 4 : 8;
-        std::vector<unsigned char> raw(7 * m->plane * rs);
-        HU_CHECK(hipMemcpy(raw.data(), m->fieldsBuf.p, raw.size(), hipMemcpyDeviceToHost));
-        const int exPlane = m->cur ? 5 : 0, hzPlane = m->cur ? 6 : 2;
+        // planes ex ey hz jx jy, from the current buffers
+        std::vector<unsigned char> raw(5 * m->plane * rs);
+        const int from[5] = {m->cur ? 5 : 0, m->cur ? 12 : 1, m->cur ? 6 : 2, 3, 4};
+        for (int pl = 0; pl < 5; ++pl)
+            HU_CHECK(hipMemcpy(raw.data() + pl * m->plane * rs, m->fieldsBuf.p + from[pl] * m->plane * rs, m->plane * rs,
+                               hipMemcpyDeviceToHost));
         // unroll the ring into logical order; planes ex ey hz/2 hz/2 jx jy
         for (int pl = 0; pl < 6; ++pl) {
-            const int src = pl == 0 ? exPlane : pl == 1 ? 1 : (pl < 4 ? hzPlane : pl - 1);
+            const int src = pl < 3 ? pl : pl - 1;
             for (int j = -mw::G; j < m->H + mw::G; ++j)
                 for (int i = -mw::G; i < m->W + mw::G; ++i) {
                     int px = (i + mw::G + h.rx) % m->Wp, py = (j + mw::G + h.ry) % m->Hp;

@@ -187,3 +187,59 @@ def test_pml_absorbs_outgoing_pulse(gpu, fp32):
         m.close()
     assert back[0] > 0.5
     assert back[16] < 5e-3
+
+
+@pytest.mark.parametrize("W,H,pml", [(16, 16, 0), (61, 17, 0), (62, 23, 0), (63, 24, 0), (64, 25, 0), (126, 31, 0),
+                                     (253, 16, 0), (254, 19, 0), (40, 17, 16), (96, 33, 16), (95, 40, 15), (160, 21, 33)])
+def test_field_step_edges(gpu, W, H, pml):
+    """Field-only steps of a window wholly inside the chamber against a numpy
+    restatement of the split step (bulk cells, guards fixed, the absorbing
+    layers' one-step psi), at window widths around the sweep's 63 columns a
+    wave and 252 a workgroup and heights around its 8-row strips.  FP64: both
+    round the same few operations per cell, so 1e-12 of the field is far above
+    their difference after 6 steps; FP32: 6 steps of about 20 roundings, 2e-5."""
+    for fp32, tol in ((False, 1e-12), (True, 2e-5)):
+        h = 1e-4
+        m = MovingWindowStep(W, H, h, h, lenBefore=1.0, lenAfter=0.1, width=0.5, phiDeg=10.0, ekinMeV=50.59, bz=0.1704,
+                             order=1, fp32=fp32, sortEvery=0, statModulus=0, cfl=0.7, pml=pml)
+        m.place(4000, 2000)
+        rng = np.random.default_rng(W + H)
+        F = np.zeros((6, H + 2, W + 2))
+        F[:2, 1:-1, 1:-1] = rng.normal(size=(2, H, W))
+        F[2, 1:-1, 1:-1] = rng.normal(size=(H, W)) / 754.0
+        F[3] = F[2]
+        m.set_fields(F)
+        m.step(6)
+        got = m.fields()
+        ex, ey, hz = F[0].copy(), F[1].copy(), F[2] + F[3]
+        # physical constants as the step uses them (Physics.cpp:41-51)
+        c = 299792458.0
+        mu0 = 1.256637061e-6
+        eps0 = 8.854187817e-12
+        dt = 0.7 * h / c
+        Z0 = np.sqrt(mu0 / eps0)
+        eta = c * dt / h
+        x = np.arange(W)
+
+        def depth(x):
+            d = np.where(x < pml, (pml - x) / max(pml, 1), 0.0)
+            return np.where(x > W - pml, (x - (W - pml)) / max(pml, 1), d)
+
+        bh, be = np.exp(-1.6 * depth(x + 0.5) ** 3 * 0.7), np.exp(-1.6 * depth(x.astype(float)) ** 3 * 0.7)
+        layer = (x < pml) | (x >= W - pml)
+        bh, be = np.where(layer, bh, 1.0), np.where(layer, be, 1.0)
+        ph, pe = np.zeros((H, W)), np.zeros((H, W))
+        c1 = (slice(1, -1), slice(1, -1))
+        for _ in range(6):
+            X = ey[1:-1, 2:] - ey[1:-1, 1:-1]
+            ph = bh * ph + (bh - 1) * X
+            for half in range(2):
+                hz[c1] += -0.5 * eta / Z0 * (X + ph) + 0.5 * eta / Z0 * (ex[2:, 1:-1] - ex[1:-1, 1:-1])
+                if half == 0:
+                    ex[c1] += eta * Z0 * (hz[1:-1, 1:-1] - hz[:-2, 1:-1])
+            d = hz[1:-1, 1:-1] - hz[1:-1, :-2]
+            pe = be * pe + (be - 1) * d
+            ey[c1] -= eta * Z0 * (d + pe)
+        for name, a, b in (("Ex", got[0], ex), ("Ey", got[1], ey), ("Hz", got[2] + got[3], hz)):
+            err = np.abs(a - b).max() / np.abs(b).max()
+            assert err < tol, (name, fp32, err)
