@@ -11,8 +11,8 @@
 // both sides are a persistent implicit GEMM on v_mfma_f32_16x16x32_bf16 with
 // LDS-staged input tiles and weights (k_conv32p); K runs over (tap, input
 // channel).  The same kernel, with transposed weights and mirrored taps, gives
-// the input gradient.  The one-channel input and output layers are load-bound
-// and run on plain vector kernels.  The weight gradient is a GEMM over pixels
+// the input gradient.  The one-channel input layer runs on the vector units, the
+// output layer (load-bound) on the MFMA.  The weight gradient is a GEMM over pixels
 // on the same MFMA, split across workgroups with FP32 atomics (k_wgrad32,
 // k_wgrad_one).  k_conv and k_conv_wgrad (16x16x16) remain for channel counts
 // the 32-channel kernels do not take.
@@ -95,7 +95,10 @@ struct ConvArgs {
     int B, H, W, Cin, Cout, CoutP;
     int flip;            // 1: taps mirrored (input gradient)
     int relu;
+    const bf16 *mask;    // [P][Cout] or null: y is zero where this is not positive (the ReLU's gradient)
 };
+
+__device__ __forceinline__ bool pos(uint32_t bits) { return __uint_as_float(bits << 16) > 0.f; }
 
 // Implicit-GEMM 3x3 convolution.  grid = (ceil(P / 256), CoutP / (16 MT));
 // each of the 4 waves covers 64 consecutive pixels of the block's 256 and MT
@@ -197,6 +200,7 @@ __global__ void __launch_bounds__(kB) k_conv(ConvArgs a)
                 if (co >= a.Cout) continue;
                 float v = acc[m][t][r] + (a.bias ? a.bias[co] : 0.f);
                 if (a.relu) v = v > 0.f ? v : 0.f;
+                if (a.mask && !pos(a.mask[p * a.Cout + co])) v = 0.f;
                 if (a.y) a.y[p * a.Cout + co] = f2bf(v);
                 if (a.yf) a.yf[p * a.Cout + co] = v;
             }
@@ -226,7 +230,6 @@ constexpr int kPIH = kPH + 2;                 // input rows with the halo
 constexpr int kPB = 512;                      // threads: 8 waves
 constexpr int kXSeg = kPIH * kIW * 4;         // 16-byte segments of one input tile chunk
 constexpr int kXPer = (kXSeg + kPB - 1) / kPB;
-constexpr int kTH = 8, kIH = kTH + 2;         // 8 x 32 pixel tiles of the one-channel layers
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
@@ -240,7 +243,9 @@ inline int conv32p_tiles(const ConvArgs &a)
     return a.B * ((a.H + kPH - 1) / kPH) * ((a.W + kTW - 1) / kTW);
 }
 
-template <int MF, int DEPTH>
+// MASK: the epilogue applies a.mask (the input gradients); without it the
+// mask's registers would cost the forward layers 2 %.
+template <int MF, int DEPTH, bool MASK>
 __global__ void __launch_bounds__(kPB, 1) k_conv32p(ConvArgs a)
 {
     constexpr int kWSeg = 9 * 16 * MF * 4;    // 16-byte segments of one weight chunk
@@ -324,6 +329,20 @@ __global__ void __launch_bounds__(kPB, 1) k_conv32p(ConvArgs a)
                 if (s < kWSeg) *reinterpret_cast<uint4 *>(&sW[(s >> 2) * kPS + 8 * seg]) = rw[j];                     \
             }                                                                                                        \
         __syncthreads();                                                                                             \
+        const bool lastChunk = (item) % nChunks == nChunks - 1;                                                      \
+        uint2 mk[MASK ? MF : 1][4];                                                                                  \
+        if (MASK && lastChunk) {           /* before the prefetch, so that their wait does not include it */         \
+            CONV32P_ORIGIN(item)                                                                                     \
+            (void)c0;                                                                                                \
+            _Pragma("unroll") for (int t = 0; t < 4; ++t)                                                            \
+            {                                                                                                        \
+                const int yy = y0 + 2 * wave + (t >> 1), xx = x0 + 16 * (t & 1) + li;                               \
+                const bool ok = yy < a.H && xx < a.W;                                                                \
+                const size_t p = ok ? ((size_t)bimg * a.H + yy) * a.W + xx : 0;                                      \
+                _Pragma("unroll") for (int m = 0; m < (MASK ? MF : 1); ++m) mk[m][t] =                               \
+                    *reinterpret_cast<const uint2 *>(a.mask + p * a.Cout + co0 + 16 * m + 4 * kg);                   \
+            }                                                                                                        \
+        }                                                                                                            \
         if ((item) + DEPTH < nItems) CONV32P_FETCH((item) + DEPTH, !wOnce, rx, rw)                                   \
         _Pragma("unroll") for (int tap = 0; tap < 9; ++tap)                                                          \
         {                                                                                                            \
@@ -339,7 +358,7 @@ __global__ void __launch_bounds__(kPB, 1) k_conv32p(ConvArgs a)
             _Pragma("unroll") for (int m = 0; m < MF; ++m)                                                           \
                 _Pragma("unroll") for (int t = 0; t < 4; ++t) acc[m][t] = mfma32(av[m], bv[t], acc[m][t]);           \
         }                                                                                                            \
-        if ((item) % nChunks == nChunks - 1) {                                                                       \
+        if (lastChunk) {                                                                                             \
             CONV32P_ORIGIN(item)                                                                                     \
             (void)c0;                                                                                                \
             _Pragma("unroll") for (int t = 0; t < 4; ++t)                                                            \
@@ -357,6 +376,13 @@ __global__ void __launch_bounds__(kPB, 1) k_conv32p(ConvArgs a)
                         if (a.relu) v[r] = v[r] > 0.f ? v[r] : 0.f;                                                  \
                     }                                                                                                \
                     acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};                                                              \
+                    if (MASK) {                                                                                      \
+                        const uint2 k = mk[MASK ? m : 0][t];                                                                    \
+                        v[0] = pos(k.x & 0xFFFFu) ? v[0] : 0.f;                                                      \
+                        v[1] = pos(k.x >> 16) ? v[1] : 0.f;                                                          \
+                        v[2] = pos(k.y & 0xFFFFu) ? v[2] : 0.f;                                                      \
+                        v[3] = pos(k.y >> 16) ? v[3] : 0.f;                                                          \
+                    }                                                                                                \
                     if (ok && a.y) {                                                                                 \
                         uint2 o;                                                                                     \
                         o.x = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);                                   \
@@ -382,8 +408,10 @@ __global__ void __launch_bounds__(kPB, 1) k_conv32p(ConvArgs a)
 
 // 3x3 convolution from one input channel to Cout (a multiple of 8, at most
 // 256) channels: one thread per pixel; the weights as floats in LDS, [tap][co],
-// read by every lane at one address.  Load-bound: 2 B in and 2 Cout B out per
-// pixel.
+// read by every lane at one address.  2 B in and 2 Cout B out per pixel, 2.4 TB/s
+// (2048 x 1024 x 4 pixels to 32 channels 224 us): the 9 Cout products, their LDS
+// reads and the strided stores bound it alike.  A thread per pixel and 8 channels,
+// whose stores are contiguous, repeats the input's loads and takes 330 us.
 __global__ void __launch_bounds__(kB) k_conv_c1(ConvArgs a)
 {
     __shared__ float sw[9 * 256];
@@ -416,60 +444,82 @@ __global__ void __launch_bounds__(kB) k_conv_c1(ConvArgs a)
         if (a.relu)
 #pragma unroll
             for (int i = 0; i < 8; ++i) o.v[i] = o.v[i] < 0.f ? 0.f : o.v[i];
+        if (a.mask) {
+            const V8 k = ld8(a.mask + (size_t)p * a.Cout + 8 * g);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o.v[i] = k.v[i] > 0.f ? o.v[i] : 0.f;
+        }
         st8(a.y + (size_t)p * a.Cout + 8 * g, o);
     }
 }
 
-// 3x3 convolution from Cin (a multiple of 32) channels to one: an 8 x 32
-// pixel tile per block of 256 threads, one pixel per thread; per chunk of 32
-// channels the tile and its halo are staged in LDS as in k_conv32, the 9 x 32
-// weights as floats.  Load-bound: 2 Cin B in and 2 (+4) B out per pixel.
+// 3x3 convolution from Cin (a multiple of 32) channels to one, as nine dot
+// products per input pixel: an MFMA with the taps as its rows (9 of 16) and 16
+// consecutive pixels as its columns, whose operand is the kilobyte those pixels
+// occupy, straight from memory.  The products of a 16 x 32 pixel tile and its
+// halo go to LDS, [tap][pixel], and each output adds its nine.  Load-bound: 2
+// Cin B in (1.2 times with the halo) and 2 (+4) B out per pixel.  With the
+// products on the vector units from an LDS copy of the input 2048 x 1024 x 4
+// pixels of 32 channels took 258 us; 124 us now.
+constexpr int kOH = 16, kOW = 32, kOBatch = 5;   // output tile, operands in flight of a wave
+constexpr int kOIW = kOW + 2, kOIH = kOH + 2, kOPix = kOIW * kOIH, kOGroups = (kOPix + 15) / 16;
 __global__ void __launch_bounds__(kB) k_conv_to1(ConvArgs a)
 {
-    __shared__ __attribute__((aligned(16))) bf16 sX[kIH * kIW * kPS];
-    __shared__ float sw[9 * 32];
-    const int tilesX = (a.W + kTW - 1) / kTW, tilesY = (a.H + kTH - 1) / kTH;
+    __shared__ float sP[9][kOGroups * 16];
+    const int tilesX = (a.W + kOW - 1) / kOW, tilesY = (a.H + kOH - 1) / kOH;
     int tile = blockIdx.x;
     const int tx = tile % tilesX;
     tile /= tilesX;
-    const int ty = tile % tilesY;
-    const int bimg = tile / tilesY;
-    const int x0 = tx * kTW, y0 = ty * kTH;
-    const int ry0 = threadIdx.x / kTW, rx0 = threadIdx.x % kTW;
-    const int Cin = a.Cin;
-    float acc = 0.f;
-    for (int c0 = 0; c0 < Cin; c0 += 32) {
-        __syncthreads();
-        for (int s = threadIdx.x; s < kIH * kIW * 4; s += kB) {
-            const int pix = s >> 2, seg = s & 3;
-            const int iy = pix / kIW, ix = pix - iy * kIW;
-            const int ys = y0 + iy - 1, xs = x0 + ix - 1;
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (ys >= 0 && ys < a.H && xs >= 0 && xs < a.W)
-                v = *reinterpret_cast<const uint4 *>(a.x + ((size_t)(bimg * a.H + ys) * a.W + xs) * Cin + c0 + 8 * seg);
-            *reinterpret_cast<uint4 *>(&sX[pix * kPS + 8 * seg]) = v;
+    const int ty = tile % tilesY, bimg = tile / tilesY;
+    const int x0 = tx * kOW, y0 = ty * kOH, Cin = a.Cin;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
+    const bf8 zero = __builtin_bit_cast(bf8, make_uint4(0u, 0u, 0u, 0u));
+    for (int g0 = wave; g0 < kOGroups; g0 += kOBatch * (kB / 64)) {
+        const bf16 *src[kOBatch];
+        bool in[kOBatch];
+        f4 acc[kOBatch];
+#pragma unroll
+        for (int k = 0; k < kOBatch; ++k) {
+            const int pix = 16 * (g0 + k * (kB / 64)) + li, ys = y0 + pix / kOIW - 1, xs = x0 + pix % kOIW - 1;
+            in[k] = pix < kOPix && ys >= 0 && ys < a.H && xs >= 0 && xs < a.W;
+            src[k] = a.x + (((size_t)bimg * a.H + ys) * a.W + xs) * Cin + 8 * kg;
+            acc[k] = f4{0.f, 0.f, 0.f, 0.f};
         }
-        for (int k = threadIdx.x; k < 9 * 32; k += kB) sw[k] = bf2f(a.w[(k >> 5) * Cin + c0 + (k & 31)]);
-        __syncthreads();
+        for (int c0 = 0; c0 < Cin; c0 += 32) {
+            // the row of the operand is the tap; rows 9 .. 15 are zero
+            const bf8 av = li < 9 ? *reinterpret_cast<const bf8 *>(a.w + li * Cin + c0 + 8 * kg) : zero;
+            bf8 bv[kOBatch];
+#pragma unroll
+            for (int k = 0; k < kOBatch; ++k) bv[k] = in[k] ? *reinterpret_cast<const bf8 *>(src[k] + c0) : zero;
+#pragma unroll
+            for (int k = 0; k < kOBatch; ++k) acc[k] = mfma32(av, bv[k], acc[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kOBatch; ++k) {
+            const int pix = 16 * (g0 + k * (kB / 64)) + li;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (4 * kg + r < 9 && pix < kOGroups * 16) sP[4 * kg + r][pix] = acc[k][r];
+        }
+    }
+    __syncthreads();
+    const float bias = a.bias ? a.bias[0] : 0.f;
+    for (int q = threadIdx.x; q < kOH * kOW; q += kB) {
+        const int ry = q / kOW, rx = q % kOW, yy = y0 + ry, xx = x0 + rx;
+        if (yy >= a.H || xx >= a.W) continue;
+        float v = 0.f;
 #pragma unroll
         for (int tap = 0; tap < 9; ++tap) {
             const int dy = a.flip ? 1 - tap / 3 : tap / 3 - 1, dx = a.flip ? 1 - tap % 3 : tap % 3 - 1;
-            const bf16 *q = &sX[((ry0 + 1 + dy) * kIW + rx0 + 1 + dx) * kPS];
-#pragma unroll
-            for (int seg = 0; seg < 4; ++seg) {
-                const V8 v = ld8(q + 8 * seg);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc += sw[tap * 32 + 8 * seg + i] * v.v[i];
-            }
+            v += sP[tap][(ry + 1 + dy) * kOIW + rx + 1 + dx];
         }
+        v += bias;
+        if (a.relu && v < 0.f) v = 0.f;
+        const size_t p = ((size_t)bimg * a.H + yy) * a.W + xx;
+        if (a.mask && !pos(a.mask[p])) v = 0.f;
+        if (a.y) a.y[p] = f2bf(v);
+        if (a.yf) a.yf[p] = v;
     }
-    const int yy = y0 + ry0, xx = x0 + rx0;
-    if (yy >= a.H || xx >= a.W) return;
-    const size_t p = ((size_t)bimg * a.H + yy) * a.W + xx;
-    float v = acc + (a.bias ? a.bias[0] : 0.f);
-    if (a.relu && v < 0.f) v = 0.f;
-    if (a.y) a.y[p] = f2bf(v);
-    if (a.yf) a.yf[p] = v;
 }
 
 // k_conv32p where the channels allow it (Cin a multiple of 32, Cout of 32);
@@ -485,15 +535,17 @@ void launch_conv(const ConvArgs &a, hipStream_t s)
             int dev = 0, cus = 0, o4 = 0, o2 = 0;
             HU_CHECK(hipGetDevice(&dev));
             HU_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-            HU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o4, k_conv32p<4, 1>, kPB, 0));
-            HU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o2, k_conv32p<2, 2>, kPB, 0));
+            HU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o4, k_conv32p<4, 1, false>, kPB, 0));
+            HU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o2, k_conv32p<2, 2, false>, kPB, 0));
             slots2 = cus * std::max(o2, 1);
             slots4 = cus * std::max(o4, 1);
         }
         const int mf = a.Cout % 64 == 0 ? 4 : 2, nCo = a.Cout / (16 * mf);
         const int G = std::max(1, std::min(conv32p_tiles(a), (mf == 4 ? slots4 : slots2) / nCo));
-        if (mf == 4) k_conv32p<4, 1><<<G * nCo, kPB, 0, s>>>(a);
-        else k_conv32p<2, 2><<<G * nCo, kPB, 0, s>>>(a);
+        if (mf == 4 && a.mask) k_conv32p<4, 1, true><<<G * nCo, kPB, 0, s>>>(a);
+        else if (mf == 4) k_conv32p<4, 1, false><<<G * nCo, kPB, 0, s>>>(a);
+        else if (a.mask) k_conv32p<2, 2, true><<<G * nCo, kPB, 0, s>>>(a);
+        else k_conv32p<2, 2, false><<<G * nCo, kPB, 0, s>>>(a);
         return;
     }
     if (a.Cin == 1 && a.Cout % 8 == 0 && a.Cout <= 256 && a.y && (double)a.B * a.H * a.W < 2e9) {
@@ -502,7 +554,7 @@ void launch_conv(const ConvArgs &a, hipStream_t s)
         return;
     }
     if (a.Cout == 1 && a.Cin % 32 == 0) {
-        k_conv_to1<<<a.B * ((a.H + kTH - 1) / kTH) * ((a.W + kTW - 1) / kTW), kB, 0, s>>>(a);
+        k_conv_to1<<<a.B * ((a.H + kOH - 1) / kOH) * ((a.W + kOW - 1) / kOW), kB, 0, s>>>(a);
         return;
     }
     const int P = a.B * a.H * a.W;
@@ -513,6 +565,8 @@ void launch_conv(const ConvArgs &a, hipStream_t s)
     else k_conv<1><<<grid, kB, 0, s>>>(a);
 }
 
+// Gradients are added with the hardware's FP32 atomic (atomicAdd compiles to a
+// compare-and-swap loop).
 // Weight gradient dW[co][tap][ci] += sum_p dY[p][co] X[p + s(tap)][ci]:
 // M = Cout, N = 9 Cin (n = tap * Cin + ci), K = pixels, split over blockIdx.z.
 // grid = (ceil(9 Cin / 64), CoutP / 16, splits); 64 threads per block.
@@ -569,7 +623,7 @@ __global__ void __launch_bounds__(64) k_conv_wgrad(const bf16 *dy, const bf16 *x
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int c = co0 + 4 * kg + r;
-            if (c < Cout) atomicAdd(&dw[(size_t)c * N + n], acc[t][r]);
+            if (c < Cout) unsafeAtomicAdd(&dw[(size_t)c * N + n], acc[t][r]);
         }
     }
 }
@@ -586,6 +640,10 @@ __global__ void __launch_bounds__(64) k_conv_wgrad(const bf16 *dy, const bf16 *x
 // reads of the input row give the three dx shifts by funnel shifts of the
 // lane's registers.  Row pitches are padded so that 16 lanes' 16-byte reads
 // fall on distinct banks.  One atomic per weight and workgroup at the end.
+// Two workgroups fit a CU, so 512 fill the chip; each more only adds its
+// 18 000 atomics: 64 to 64 channels over 256 x 256 x 4 pixels take 102 us with
+// 1024 workgroups, 77 with 512, 92 with 256.
+constexpr int kWgBlocks = 512;
 constexpr int kWgTH = 8, kWgTW = 32;          // pixel tile
 constexpr int kDyPitch = kWgTH * kWgTW + 8;   // bf16 per output channel in LDS
 constexpr int kXCols = 40;                    // input columns x0 - 1 .. x0 + 38
@@ -596,8 +654,8 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ bf8 as_bf8(u4v v) { return __builtin_bit_cast(bf8, v); }
 
 template <int CF, int WCO>
-__global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x, float *dw, int B, int H, int W,
-                                                   int Cin, int Cout, int ksplit)
+__global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x, float *dw, float *db, int B, int H,
+                                                   int W, int Cin, int Cout, int ksplit)
 {
     constexpr int CO_BLK = 16 * CF * WCO, CI_BLK = 16 * (4 / WCO);
     __shared__ __attribute__((aligned(16))) bf16 sD[CO_BLK * kDyPitch];
@@ -614,6 +672,10 @@ __global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x
     for (int m = 0; m < CF; ++m)
 #pragma unroll
         for (int t = 0; t < 9; ++t) acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};
+    // the bias gradient, from the dY that is staged anyway (one block of input
+    // channels does it): this thread always stages channels co0 + 8 (tid % (CO_BLK / 8))
+    const bool bias = ci0 == 0;
+    float bs[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int tile = kz; tile < nTiles; tile += ksplit) {
         const int tx = tile % tilesX, rest = tile / tilesX;
         const int x0 = tx * kWgTW, y0 = (rest % tilesY) * kWgTH, bimg = rest / tilesY;
@@ -639,6 +701,7 @@ __global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x
                 };
                 const uint2 o = make_uint2(h(v[0]) | (h(v[1]) << 16), h(v[2]) | (h(v[3]) << 16));
                 *reinterpret_cast<uint2 *>(&sD[(8 * cg + e) * kDyPitch + r * kWgTW + 4 * x4]) = o;
+                if (bias) bs[e] += (bf2f(h(v[0])) + bf2f(h(v[1]))) + (bf2f(h(v[2])) + bf2f(h(v[3])));
             }
         }
         // input with its halo: units (row, 4-column group, 8-channel group)
@@ -690,6 +753,19 @@ __global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x
             }
         }
     }
+    if (bias) {
+        __syncthreads();
+        float *sb = reinterpret_cast<float *>(sD);     // [256][8]
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sb[tid * 8 + e] = bs[e];
+        __syncthreads();
+        if (tid < CO_BLK) {
+            const int g = tid / 8, e = tid % 8;
+            float t = 0.f;
+            for (int q = g; q < kB; q += CO_BLK / 8) t += sb[q * 8 + e];
+            unsafeAtomicAdd(&db[co0 + tid], t);
+        }
+    }
     // D[4 kg + rr][li]: output channel co0 + 16 (cf0 + m) + 4 kg + rr, input channel ci0 + 16 nf + li
     const int ci = ci0 + 16 * nf + li;
 #pragma unroll
@@ -699,7 +775,7 @@ __global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
                 const int co = co0 + 16 * (cf0 + m) + 4 * kg + rr;
-                atomicAdd(&dw[((size_t)co * 9 + t) * Cin + ci], acc[m][t][rr]);
+                unsafeAtomicAdd(&dw[((size_t)co * 9 + t) * Cin + ci], acc[m][t][rr]);
             }
 }
 
@@ -710,7 +786,7 @@ __global__ void __launch_bounds__(kB, 2) k_wgrad32(const bf16 *dy, const bf16 *x
 // w & 1 of the 32-channel side and tile rows (w >> 1) + 2 j.  Staging and
 // shifts as in k_wgrad32; pixel tiles blockIdx.x, + gridDim.x, ...
 template <bool OUT1>
-__global__ void __launch_bounds__(kB) k_wgrad_one(const bf16 *dy, const bf16 *x, float *dw, int B, int H, int W)
+__global__ void __launch_bounds__(kB) k_wgrad_one(const bf16 *dy, const bf16 *x, float *dw, float *db, int B, int H, int W)
 {
     constexpr int NCO = OUT1 ? 1 : 32, NCI = OUT1 ? 32 : 1;
     __shared__ __attribute__((aligned(16))) bf16 sD[NCO * kDyPitch];
@@ -722,6 +798,7 @@ __global__ void __launch_bounds__(kB) k_wgrad_one(const bf16 *dy, const bf16 *x,
 #pragma unroll
     for (int t = 0; t < 9; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
     const u4v zero = {0u, 0u, 0u, 0u};
+    float bs[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // bias gradient, as in k_wgrad32
     for (int tile = blockIdx.x; tile < nTiles; tile += gridDim.x) {
         const int tx = tile % tilesX, rest = tile / tilesX;
         const int x0 = tx * kWgTW, y0 = (rest % tilesY) * kWgTH, bimg = rest / tilesY;
@@ -737,6 +814,7 @@ __global__ void __launch_bounds__(kB) k_wgrad_one(const bf16 *dy, const bf16 *x,
                 for (int q = 0; q < 4; ++q) {
                     const int xx = x0 + 4 * x4 + q;
                     h[q] = (yy < H && xx < W) ? (uint32_t)dy[((size_t)bimg * H + yy) * W + xx] : 0u;
+                    bs[0] += bf2f((bf16)h[q]);
                 }
                 *reinterpret_cast<uint2 *>(&sD[r * kWgTW + 4 * x4]) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
             } else {
@@ -756,6 +834,7 @@ __global__ void __launch_bounds__(kB) k_wgrad_one(const bf16 *dy, const bf16 *x,
                     };
                     *reinterpret_cast<uint2 *>(&sD[(8 * cg + e) * kDyPitch + r * kWgTW + 4 * x4]) =
                         make_uint2(h(v[0]) | (h(v[1]) << 16), h(v[2]) | (h(v[3]) << 16));
+                    bs[e] += (bf2f(h(v[0])) + bf2f(h(v[1]))) + (bf2f(h(v[2])) + bf2f(h(v[3])));
                 }
             }
         }
@@ -821,49 +900,42 @@ __global__ void __launch_bounds__(kB) k_wgrad_one(const bf16 *dy, const bf16 *x,
             }
         }
     }
+    // The workgroup's sums meet in LDS, one atomic per weight and workgroup: all
+    // workgroups add into the same 288 weights, and with an atomic per wave the
+    // additions to one address took longer than the products.
     // D[4 kg + rr][li]: row = output channel (OUT1: only row 0), column = input channel (else: only column 0)
+    __shared__ float sw[288], sb[kB * (OUT1 ? 1 : 8)];
+    for (int q = tid; q < 288; q += kB) sw[q] = 0.f;
+#pragma unroll
+    for (int e = 0; e < (OUT1 ? 1 : 8); ++e) sb[tid * (OUT1 ? 1 : 8) + e] = bs[e];
+    __syncthreads();
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
         if (OUT1) {
-            if (kg == 0) atomicAdd(&dw[t * 32 + 16 * fr + li], acc[t][0]);
+            if (kg == 0) unsafeAtomicAdd(&sw[t * 32 + 16 * fr + li], acc[t][0]);
         } else if (li == 0) {
 #pragma unroll
-            for (int rr = 0; rr < 4; ++rr) atomicAdd(&dw[(16 * fr + 4 * kg + rr) * 9 + t], acc[t][rr]);
+            for (int rr = 0; rr < 4; ++rr) unsafeAtomicAdd(&sw[(16 * fr + 4 * kg + rr) * 9 + t], acc[t][rr]);
         }
+    }
+    __syncthreads();
+    for (int q = tid; q < 288; q += kB) unsafeAtomicAdd(&dw[q], sw[q]);
+    if (tid < NCO) {
+        float t = 0.f;
+        if (OUT1) {
+            for (int q = 0; q < kB; ++q) t += sb[q];
+        } else {
+            for (int q = tid / 8; q < kB; q += NCO / 8) t += sb[q * 8 + tid % 8];
+        }
+        unsafeAtomicAdd(&db[tid], t);
     }
 }
 
 // Elementwise kernels take 8 channels (one 16-byte vector) per thread: every
 // activation they touch has a channel count that is a multiple of 8.
 
-// bias gradient: db[co] += sum_p dY[p][co].  Thread t of a block reads the 8
-// channels 8 (t % (C/8)) of pixels t / (C/8) + k 256 / (C/8); the partial
-// sums of one channel group meet in LDS, one atomic per channel and block.
-// C a multiple of 8 dividing 2048.
-__global__ void __launch_bounds__(kB) k_bias_grad8(const bf16 *dy, float *db, int P, int C)
-{
-    __shared__ float sh[kB][9];
-    const int groups = C / 8, cg = threadIdx.x % groups, row = threadIdx.x / groups, rows = kB / groups;
-    V8 s;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) s.v[i] = 0.f;
-    for (int p = blockIdx.x * rows + row; p < P; p += gridDim.x * rows) {
-        const V8 v = ld8(dy + (size_t)p * C + 8 * cg);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s.v[i] += v.v[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sh[threadIdx.x][i] = s.v[i];
-    __syncthreads();
-    if ((int)threadIdx.x < C) {
-        const int g = threadIdx.x / 8, i = threadIdx.x % 8;
-        float t = 0.f;
-        for (int r = 0; r < rows; ++r) t += sh[r * groups + g][i];
-        atomicAdd(&db[threadIdx.x], t);
-    }
-}
-
-// bias gradient for any C (the 1-channel output layer): one block per channel
+// bias gradient for any C (layers whose weight gradient runs on k_conv_wgrad):
+// one block per channel
 __global__ void k_bias_grad(const bf16 *dy, float *db, int P, int C)
 {
     __shared__ float sh[kB];
@@ -876,24 +948,7 @@ __global__ void k_bias_grad(const bf16 *dy, float *db, int P, int C)
         if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(&db[c], sh[0]);
-}
-
-// dPre = dY * (Y > 0); n8 = elements / 8
-__global__ void k_relu_grad(const bf16 *dy, const bf16 *y, bf16 *out, size_t n8)
-{
-    const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (k >= n8) return;
-    const uint4 g = reinterpret_cast<const uint4 *>(dy)[k], a = reinterpret_cast<const uint4 *>(y)[k];
-    const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, aw[4] = {a.x, a.y, a.z, a.w};
-    uint32_t o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t lo = __uint_as_float(aw[i] << 16) > 0.f ? 0x0000FFFFu : 0u;
-        const uint32_t hi = __uint_as_float(aw[i] & 0xFFFF0000u) > 0.f ? 0xFFFF0000u : 0u;
-        o[i] = gw[i] & (lo | hi);
-    }
-    reinterpret_cast<uint4 *>(out)[k] = make_uint4(o[0], o[1], o[2], o[3]);
+    if (threadIdx.x == 0) unsafeAtomicAdd(&db[c], sh[0]);
 }
 
 // 2x2 average pool (NHWC); H, W even; one thread per output pixel and 8 channels
@@ -915,7 +970,10 @@ __global__ void k_pool(const bf16 *x, bf16 *y, int B, int H, int W, int C)
     st8(y + k * 8, o);
 }
 
-__global__ void k_pool_grad(const bf16 *dy, bf16 *dx, int B, int H, int W, int C)
+// Gradient at a skip activation y (a ReLU output that is pooled and also added to
+// the decoder): dx = pool^T(dy) + ds where y is positive, 0 elsewhere.  0.25 dy
+// is exact in bf16, so one rounding is left.
+__global__ void k_skip_grad(const bf16 *dy, const bf16 *ds, const bf16 *y, bf16 *dx, int B, int H, int W, int C)
 {
     const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
     const int C8 = C / 8;
@@ -926,8 +984,9 @@ __global__ void k_pool_grad(const bf16 *dy, bf16 *dx, int B, int H, int W, int C
     const int yy = (int)(r % H);
     const int b = (int)(r / H);
     V8 o = ld8(dy + (((size_t)b * (H / 2) + yy / 2) * (W / 2) + xx / 2) * C + c);
+    const V8 t = ld8(ds + k * 8), a = ld8(y + k * 8);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o.v[i] *= 0.25f;
+    for (int i = 0; i < 8; ++i) o.v[i] = a.v[i] > 0.f ? 0.25f * o.v[i] + t.v[i] : 0.f;
     st8(dx + k * 8, o);
 }
 
@@ -949,8 +1008,9 @@ __global__ void k_up_add(const bf16 *x, const bf16 *s, bf16 *y, int B, int H, in
     st8(y + k * 8, o);
 }
 
-// gradient of up(x): dx[y][x] = sum of the 2x2 block of dy
-__global__ void k_up_grad(const bf16 *dy, bf16 *dx, int B, int Hs, int Ws, int C)
+// gradient of up(x) at a ReLU output x: dx[y][x] = sum of the 2x2 block of dy
+// where x is positive, 0 elsewhere
+__global__ void k_up_grad(const bf16 *dy, const bf16 *x, bf16 *dx, int B, int Hs, int Ws, int C)
 {
     const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
     const int C8 = C / 8;
@@ -964,21 +1024,10 @@ __global__ void k_up_grad(const bf16 *dy, bf16 *dx, int B, int Hs, int Ws, int C
     const bf16 *q = dy + (((size_t)b * 2 * Hs + 2 * yy) * W + 2 * xx) * C + c;
     const V8 a = ld8(q), bb = ld8(q + C), cc = ld8(q + (size_t)W * C), d = ld8(q + (size_t)W * C + C);
     V8 o;
+    const V8 xv = ld8(x + k * 8);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o.v[i] = a.v[i] + bb.v[i] + cc.v[i] + d.v[i];
+    for (int i = 0; i < 8; ++i) o.v[i] = xv.v[i] > 0.f ? a.v[i] + bb.v[i] + cc.v[i] + d.v[i] : 0.f;
     st8(dx + k * 8, o);
-}
-
-// y = a + b; n8 = elements / 8
-__global__ void k_add_bf(const bf16 *a, const bf16 *b, bf16 *y, size_t n8)
-{
-    const size_t k = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (k >= n8) return;
-    V8 o = ld8(a + 8 * k);
-    const V8 t = ld8(b + 8 * k);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o.v[i] += t.v[i];
-    st8(y + 8 * k, o);
 }
 
 __global__ void k_to_bf(const float *x, bf16 *y, size_t n, float scale)
@@ -1005,7 +1054,7 @@ __global__ void k_mse(const float *o, const float *t, bf16 *g, float *loss, size
         if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(loss, sh[0] / (float)n);
+    if (threadIdx.x == 0) unsafeAtomicAdd(loss, sh[0] / (float)n);
 }
 
 // Adam on the fp32 master weights; refresh the bf16 copies (padded rows stay 0)
@@ -1116,17 +1165,18 @@ void conv(csrst_warmstart *u, int li, const bf16 *x, bf16 *y, float *yf, int B, 
     const Layer &l = u->L[li];
     ConvArgs a;
     a.x = x; a.w = u->wb.p + u->wbOff[li]; a.bias = u->w.p + l.boff; a.y = y; a.yf = yf;
-    a.B = B; a.H = H; a.W = W; a.Cin = l.cin; a.Cout = l.cout; a.CoutP = pad16(l.cout); a.flip = 0; a.relu = l.relu;
+    a.B = B; a.H = H; a.W = W; a.Cin = l.cin; a.Cout = l.cout; a.CoutP = pad16(l.cout); a.flip = 0; a.relu = l.relu; a.mask = nullptr;
     launch_conv(a, u->s);
 }
 
-// input gradient of conv li: dx[P][cin] from dpre[P][cout]
-void conv_dgrad(csrst_warmstart *u, int li, const bf16 *dpre, bf16 *dx, int B, int H, int W)
+// input gradient of conv li: dx[P][cin] from dpre[P][cout], zero where mask (the
+// input, if a ReLU made it) is not positive
+void conv_dgrad(csrst_warmstart *u, int li, const bf16 *dpre, bf16 *dx, const bf16 *mask, int B, int H, int W)
 {
     const Layer &l = u->L[li];
     ConvArgs a;
     a.x = dpre; a.w = u->wt.p + u->wtOff[li]; a.bias = nullptr; a.y = dx; a.yf = nullptr;
-    a.B = B; a.H = H; a.W = W; a.Cin = l.cout; a.Cout = l.cin; a.CoutP = pad16(l.cin); a.flip = 1; a.relu = 0;
+    a.B = B; a.H = H; a.W = W; a.Cin = l.cout; a.Cout = l.cin; a.CoutP = pad16(l.cin); a.flip = 1; a.relu = 0; a.mask = mask;
     launch_conv(a, u->s);
 }
 
@@ -1140,22 +1190,19 @@ void conv_wgrad(csrst_warmstart *u, int li, const bf16 *dpre, const bf16 *x, int
         const int tiles = B * ((H + kWgTH - 1) / kWgTH) * ((W + kWgTW - 1) / kWgTW);
         auto go = [&](auto kern, int coBlk, int ciBlk) {
             const int nBlk = (l.cout / coBlk) * (l.cin / ciBlk);
-            const int ksplit = std::max(1, std::min(tiles, 1024 / nBlk));
-            kern<<<nBlk * ksplit, kB, 0, u->s>>>(dpre, x, u->g.p + l.woff, B, H, W, l.cin, l.cout, ksplit);
+            const int ksplit = std::max(1, std::min(tiles, kWgBlocks / nBlk));
+            kern<<<nBlk * ksplit, kB, 0, u->s>>>(dpre, x, u->g.p + l.woff, u->g.p + l.boff, B, H, W, l.cin, l.cout, ksplit);
         };
         if (l.cin % 64 == 0) go(k_wgrad32<2, 1>, 32, 64);
         else if (l.cout % 64 == 0) go(k_wgrad32<2, 2>, 64, 32);
         else go(k_wgrad32<1, 2>, 32, 32);
     } else if ((l.cin == 1 && l.cout == 32) || (l.cin == 32 && l.cout == 1)) {
         const int tiles = B * ((H + kWgTH - 1) / kWgTH) * ((W + kWgTW - 1) / kWgTW);
-        if (l.cout == 1) k_wgrad_one<true><<<std::min(tiles, 1024), kB, 0, u->s>>>(dpre, x, u->g.p + l.woff, B, H, W);
-        else k_wgrad_one<false><<<std::min(tiles, 1024), kB, 0, u->s>>>(dpre, x, u->g.p + l.woff, B, H, W);
-    } else
-        k_conv_wgrad<<<grid, 64, 0, u->s>>>(dpre, x, u->g.p + l.woff, B, H, W, l.cin, l.cout, chunk);
-    if (l.cout % 8 == 0 && kB % (l.cout / 8) == 0) {
-        const int rows = kB / (l.cout / 8);
-        k_bias_grad8<<<std::min(1024, (P + rows - 1) / rows), kB, 0, u->s>>>(dpre, u->g.p + l.boff, P, l.cout);
+        float *w = u->g.p + l.woff, *b = u->g.p + l.boff;
+        if (l.cout == 1) k_wgrad_one<true><<<std::min(tiles, 1024), kB, 0, u->s>>>(dpre, x, w, b, B, H, W);
+        else k_wgrad_one<false><<<std::min(tiles, 1024), kB, 0, u->s>>>(dpre, x, w, b, B, H, W);
     } else {
+        k_conv_wgrad<<<grid, 64, 0, u->s>>>(dpre, x, u->g.p + l.woff, B, H, W, l.cin, l.cout, chunk);
         dim3 bg(std::min(64, (P + kB - 1) / kB), l.cout);
         k_bias_grad<<<bg, kB, 0, u->s>>>(dpre, u->g.p + l.boff, P, l.cout);
     }
@@ -1195,11 +1242,6 @@ void plan(csrst_warmstart *u, int B)
     for (auto &e : sh) add(u->A, e[0], e[1], e[2]);
     u->Gd.clear();
     for (auto &e : sh) add(u->Gd, e[0], e[1], e[2]);
-    // two scratch gradient buffers of the largest activation
-    size_t big = 0;
-    for (auto &e : sh) big = std::max(big, (size_t)B * e[0] * e[1] * e[2]);
-    u->Gd.push_back({off, 0, 0, 0}); off += (big + 63) / 64 * 64;
-    u->Gd.push_back({off, 0, 0, 0}); off += (big + 63) / 64 * 64;
     // grow only: a smaller batch reuses the arena with its own offsets
     if (off > u->act.n) u->act.alloc(off);
     if ((size_t)B * H * W > u->outf.n) u->outf.alloc((size_t)B * H * W);
@@ -1252,34 +1294,23 @@ void backward(csrst_warmstart *u, int B)
     const int H = u->H, W = u->W;
     auto P = [&](int i) { return u->ptr(A[i]); };
     auto D = [&](int i) { return u->ptr(G[i]); };
-    bf16 *pre = u->ptr(G[22]);
     HU_CHECK(hipMemsetAsync(u->g.p, 0, u->nparam * sizeof(float), u->s));
-    // conv li with input activation xin and output activation yout; dy given in D(yout)
+    // conv li with input activation xin and output activation yout.  D(yout) is
+    // the gradient before the ReLU: whatever produces a gradient at a ReLU's
+    // output masks it there.
     auto back = [&](int li, int xin, int yout, int h, int w, bool needDx) {
-        const Layer &l = u->L[li];
-        const size_t n = (size_t)B * h * w * l.cout;
-        const bf16 *dpre = D(yout);
-        if (l.relu) {
-            k_relu_grad<<<nb(n / 8), kB, 0, u->s>>>(D(yout), P(yout), pre, n / 8);
-            dpre = pre;
-        }
-        conv_wgrad(u, li, dpre, P(xin), B, h, w);
-        if (needDx) conv_dgrad(u, li, dpre, D(xin), B, h, w);
-    };
-    auto addgrad = [&](int dst, const bf16 *src) {   // D(dst) += src
-        const auto &d = A[dst];
-        const size_t n = (size_t)B * d.h * d.w * d.c;
-        k_add_bf<<<nb(n / 8), kB, 0, u->s>>>(D(dst), src, D(dst), n / 8);
+        const bool relu = xin == 20 || xin == 17 || xin == 14 || xin == 11 || xin == 10 || xin == 7 || xin == 4 || xin == 1;
+        conv_wgrad(u, li, D(yout), P(xin), B, h, w);
+        if (needDx) conv_dgrad(u, li, D(yout), D(xin), relu ? P(xin) : nullptr, B, h, w);
     };
     auto upgrad = [&](int dstLow, int srcHigh) {      // D(dstLow) = up^T D(srcHigh)
         const auto &d = A[dstLow];
-        k_up_grad<<<nb((size_t)B * d.h * d.w * d.c / 8), kB, 0, u->s>>>(D(srcHigh), D(dstLow), B, d.h, d.w, d.c);
+        k_up_grad<<<nb((size_t)B * d.h * d.w * d.c / 8), kB, 0, u->s>>>(D(srcHigh), P(dstLow), D(dstLow), B, d.h, d.w, d.c);
     };
-    auto poolgrad = [&](bf16 *dst, int srcLow, int hiIdx) {   // dst = pool^T D(srcLow)
-        const auto &d = A[hiIdx];
-        k_pool_grad<<<nb((size_t)B * d.h * d.w * d.c / 8), kB, 0, u->s>>>(D(srcLow), dst, B, d.h, d.w, d.c);
+    auto skipgrad = [&](int at, int low, int dec) {    // D(at) = pool^T D(low) + D(dec)
+        const auto &d = A[at];
+        k_skip_grad<<<nb((size_t)B * d.h * d.w * d.c / 8), kB, 0, u->s>>>(D(low), D(dec), P(at), D(at), B, d.h, d.w, d.c);
     };
-    bf16 *tmp = u->ptr(G[23]);
     back(14, 20, 21, H, W, true);      // out -> D20
     back(13, 19, 20, H, W, true);      // -> D19 (= d(up(c02)) and d(s0))
     upgrad(18, 19);                    // D18 = up^T D19
@@ -1292,20 +1323,15 @@ void backward(csrst_warmstart *u, int B)
     back(8, 11, 12, H / 8, W / 8, true);
     back(7, 10, 11, H / 8, W / 8, true);
     back(6, 9, 10, H / 8, W / 8, true);
-    // D8 = pool^T D9 + D13 (skip)
-    poolgrad(D(8), 9, 8);
-    addgrad(8, D(13));
+    skipgrad(8, 9, 13);
     back(5, 7, 8, H / 4, W / 4, true);
     back(4, 6, 7, H / 4, W / 4, true);
-    poolgrad(D(5), 6, 5);
-    addgrad(5, D(16));
+    skipgrad(5, 6, 16);
     back(3, 4, 5, H / 2, W / 2, true);
     back(2, 3, 4, H / 2, W / 2, true);
-    poolgrad(D(2), 3, 2);
-    addgrad(2, D(19));
+    skipgrad(2, 3, 19);
     back(1, 1, 2, H, W, true);
     back(0, 0, 1, H, W, false);
-    (void)tmp;
     HU_LAUNCH_CHECK();
 }
 

@@ -46,6 +46,28 @@ def test_forward_and_gradients_match_cpu(gpu, H, W, B):
         assert e < 6e-2, (i, e)
 
 
+@pytest.mark.parametrize("H,W,B", [(16, 16, 1), (24, 40, 1), (16, 136, 3), (56, 64, 1)])
+def test_gradients_at_tile_edges(gpu, H, W, B):
+    """Rectangles that end inside the 8 x 32 and 16 x 32 pixel tiles of the
+    convolution and weight-gradient kernels, at the top level and below (56 x
+    64 gives 7 x 8 at the bottom): every ReLU mask, skip and pooling gradient
+    and bias sum against the CPU.  A BF16 rounding is 2^-9; about 30 of them
+    follow one another and add as a random walk to 1e-2 of a layer's norm,
+    bounded here at six times that."""
+    rng = np.random.default_rng(H + W)
+    u = WarmStart(H, W, max_batch=B)
+    rho = rng.normal(size=(B, H, W)).astype(np.float32)
+    phi = rng.normal(size=(B, H, W)).astype(np.float32)
+    ref = Ref(u.weights())
+    want = ref.forward(rho)
+    gw = ref.backward(want, phi)
+    assert rel(u.infer(rho), want) < 6e-2
+    _, g = u.gradients(rho, phi)
+    for i, l in enumerate(layers()[0]):
+        sl = slice(l["woff"], l["boff"] + l["cout"])
+        assert rel(g[sl], gw[sl]) < 6e-2, (i, rel(g[sl], gw[sl]))
+
+
 def make_sample(rng, H, W, h):
     """1-4 Gaussians (sigma 40-500 um) summing to one charge unit, on an
     H x W grid of spacing h inside a rectangular chamber (edges grounded)."""
