@@ -943,13 +943,13 @@ extern "C" int csrst_poisson_solve(int nx, int ny, double hx, double hy, const u
         DBuf<double> db, dphi;
         dcls.alloc(m); db.alloc(m); dphi.alloc(m);
         HU_CHECK(hipMemcpyAsync(dcls.p, cls, m, hipMemcpyHostToDevice, s));
-        HU_CHECK(hipMemcpyAsync(db.p, b, m * sizeof(double), hipMemcpyHostToDevice, s));
-        HU_CHECK(hipMemcpyAsync(dphi.p, phi, m * sizeof(double), hipMemcpyHostToDevice, s));
+        hu::Stage stage;
+        stage.in(db.p, b, m * sizeof(double), s);
+        stage.in(dphi.p, phi, m * sizeof(double), s);
         pmg::Solver sol;
         sol.setup(nx, ny, hx, hy, dcls.p, s);
         const pmg::Stats st = sol.solve(db.p, dphi.p, tol, maxit);
-        HU_CHECK(hipMemcpyAsync(phi, dphi.p, m * sizeof(double), hipMemcpyDeviceToHost, s));
-        HU_CHECK(hipStreamSynchronize(s));
+        stage.out(phi, dphi.p, m * sizeof(double), s);
         HU_CHECK(hipStreamDestroy(s));
         s = nullptr;
         if (cycles) *cycles = st.cycles;

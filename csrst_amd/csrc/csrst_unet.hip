@@ -1104,6 +1104,7 @@ struct csrst_warmstart {
     std::string err;
     hipStream_t s = nullptr;
     int H = 0, W = 0, base = 32, maxBatch = 0;
+    hu::Stage stage;     // transfers on s of arrays in pageable memory
     std::vector<Layer> L;          // 15 convolutions
     size_t nparam = 0;
     DBuf<float> w, m, v, g;        // master weights, Adam moments, gradients
@@ -1339,7 +1340,7 @@ void upload_input(csrst_warmstart *u, const float *rho, int B, float scale)
 {
     const size_t n = (size_t)B * u->H * u->W;
     u->scratchF.alloc(std::max(u->scratchF.n, n));
-    HU_CHECK(hipMemcpyAsync(u->scratchF.p, rho, n * sizeof(float), hipMemcpyHostToDevice, u->s));
+    u->stage.in(u->scratchF.p, rho, n * sizeof(float), u->s);
     k_to_bf<<<nb(n), kB, 0, u->s>>>(u->scratchF.p, u->ptr(u->A[0]), n, scale);
     HU_LAUNCH_CHECK();
 }
@@ -1767,8 +1768,7 @@ int csrst_warmstart_infer(csrst_warmstart *u, const float *rho, float *out, int 
         plan(u, B);
         upload_input(u, rho, B, scale);
         forward(u, B);
-        HU_CHECK(hipMemcpyAsync(out, u->outf.p, (size_t)B * u->H * u->W * sizeof(float), hipMemcpyDeviceToHost, u->s));
-        HU_CHECK(hipStreamSynchronize(u->s));
+        u->stage.out(out, u->outf.p, (size_t)B * u->H * u->W * sizeof(float), u->s);
         return CSRST_OK;
     } catch (const std::exception &e) {
         return ws_fail(u, e);
@@ -1785,13 +1785,13 @@ int csrst_warmstart_gradients(csrst_warmstart *u, const float *rho, const float 
         plan(u, B);
         upload_input(u, rho, B, scale);
         const size_t np = (size_t)B * u->H * u->W;
-        HU_CHECK(hipMemcpyAsync(u->tgt.p, phi, np * sizeof(float), hipMemcpyHostToDevice, u->s));
+        u->stage.in(u->tgt.p, phi, np * sizeof(float), u->s);
         forward(u, B);
         HU_CHECK(hipMemsetAsync(u->lossBuf.p, 0, sizeof(float), u->s));
         k_mse<<<std::min(nb(np), kMseBlocks), kB, 0, u->s>>>(u->outf.p, u->tgt.p, u->ptr(u->Gd[21]), u->lossBuf.p, np);
         backward(u, B);
         if (loss) HU_CHECK(hipMemcpyAsync(loss, u->lossBuf.p, sizeof(float), hipMemcpyDeviceToHost, u->s));
-        if (grads) HU_CHECK(hipMemcpyAsync(grads, u->g.p, u->nparam * sizeof(float), hipMemcpyDeviceToHost, u->s));
+        if (grads) u->stage.out(grads, u->g.p, u->nparam * sizeof(float), u->s);
         HU_CHECK(hipStreamSynchronize(u->s));
         return CSRST_OK;
     } catch (const std::exception &e) {
@@ -1835,8 +1835,8 @@ int csrst_warmstart_solve(csrst_warmstart *u, double hx, double hy, const uint8_
         loop_grid(u, hx, hy, cls);
         auto &Lp = u->loop;
         const size_t n = (size_t)u->H * u->W;
-        HU_CHECK(hipMemcpyAsync(Lp.b.p, b, n * sizeof(double), hipMemcpyHostToDevice, u->s));
-        HU_CHECK(hipMemcpyAsync(Lp.phi.p, phi, n * sizeof(double), hipMemcpyHostToDevice, u->s));
+        u->stage.in(Lp.b.p, b, n * sizeof(double), u->s);
+        u->stage.in(Lp.phi.p, phi, n * sizeof(double), u->s);
         const double bn = Lp.mg.begin(Lp.b.p, Lp.phi.p);
         double r = Lp.mg.resnorm();
         const double target = tol * (bn > 0 ? bn : 1.0);
@@ -1851,8 +1851,7 @@ int csrst_warmstart_solve(csrst_warmstart *u, double hx, double hy, const uint8_
             r = rn;
         }
         Lp.mg.store(Lp.b.p, Lp.phi.p);
-        HU_CHECK(hipMemcpyAsync(phi, Lp.phi.p, n * sizeof(double), hipMemcpyDeviceToHost, u->s));
-        HU_CHECK(hipStreamSynchronize(u->s));
+        u->stage.out(phi, Lp.phi.p, n * sizeof(double), u->s);
         if (cycles) *cycles = cyc;
         if (resid) *resid = bn > 0 ? r / bn : r;
         return CSRST_OK;
@@ -1885,7 +1884,7 @@ int csrst_warmstart_train_iterates(csrst_warmstart *u, double hx, double hy, con
         int slot = 0, used = 0, nsteps = 0;
         double lsum = 0.0;
         for (int i = 0; i < nrhs; ++i) {
-            HU_CHECK(hipMemcpyAsync(Lp.b.p, b + (size_t)i * n, n * sizeof(double), hipMemcpyHostToDevice, u->s));
+            u->stage.in(Lp.b.p, b + (size_t)i * n, n * sizeof(double), u->s);
             k_zero_d<<<nb(n), kB, 0, u->s>>>(Lp.phi.p, n);
             HU_LAUNCH_CHECK();
             const double bn = Lp.mg.begin(Lp.b.p, Lp.phi.p);

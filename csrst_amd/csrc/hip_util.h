@@ -4,11 +4,15 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <thread>
+#include <vector>
 
 namespace hu {
 
@@ -73,6 +77,136 @@ struct DBuf {
     }
     void zero(hipStream_t s) { if (n) HU_CHECK(hipMemsetAsync(p, 0, n * sizeof(T), s)); }
     size_t bytes() const { return n * sizeof(T); }
+};
+
+// Copies between pageable host memory and the device through pinned buffers.
+//
+// The runtime's own path copies 13 GB/s (33.5 MB in 2.4 ms): one thread at a
+// time moves the data to or from pinned memory, page faults of a fresh result
+// array included.  Here kThreads threads do, each with two buffers of its own,
+// so that one is filled or emptied while the other is on the link.
+// 4 x 1024 x 2048 floats in and out: 4.9 ms before, 3.8 now, and no faster with 6
+// or 8 threads or with chunks of 0.5 or 2 MiB: the transfers themselves bound it.
+// Transfers below kMin stay with the runtime: a call that makes its own Stage
+// pays for the buffers too (a Poisson solve's three arrays of 4 MiB 0.07 ms slower,
+// of 11.4 MiB 0.07 ms faster, of 16 MiB 0.4, of 64 MiB 1.5).  So does host
+// memory that is already pinned.
+//
+// One Stage serves one stream at a time: it belongs to the object or call whose
+// transfers it makes and frees its buffers (8 MiB) with it.
+class Stage {
+public:
+    Stage() = default;
+    Stage(const Stage &) = delete;
+    Stage &operator=(const Stage &) = delete;
+    ~Stage()
+    {
+        for (Slot &t : slot_)
+            if (t.ev) {
+                (void)hipEventSynchronize(t.ev);
+                (void)hipEventDestroy(t.ev);
+            }
+        if (pin_) (void)hipHostFree(pin_);
+    }
+    // dst (device) = src (host); src may be reused when the call returns
+    void in(void *dst, const void *src, size_t bytes, hipStream_t s)
+    {
+        if (!staged(src, bytes)) {
+            HU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+            return;
+        }
+        run(bytes, [=](Slot *two, std::atomic<size_t> &next) -> hipError_t {
+            hipError_t e = hipSuccess;
+            size_t k;
+            for (int i = 0; (k = next.fetch_add(1)) * kChunk < bytes; i ^= 1) {
+                const size_t n = std::min(kChunk, bytes - k * kChunk);
+                if ((e = hipEventSynchronize(two[i].ev)) != hipSuccess) return e;   // its last transfer has ended
+                memcpy(two[i].p, (const char *)src + k * kChunk, n);
+                if ((e = hipMemcpyAsync((char *)dst + k * kChunk, two[i].p, n, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+                if ((e = hipEventRecord(two[i].ev, s)) != hipSuccess) return e;
+            }
+            return e;
+        });
+    }
+    // dst (host) = src (device) as the stream's work so far leaves it; complete when the call returns
+    void out(void *dst, const void *src, size_t bytes, hipStream_t s)
+    {
+        if (!staged(dst, bytes)) {
+            HU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+            HU_CHECK(hipStreamSynchronize(s));
+            return;
+        }
+        run(bytes, [=](Slot *two, std::atomic<size_t> &next) -> hipError_t {
+            hipError_t e = hipSuccess;
+            size_t at[2] = {bytes, bytes};                                          // offsets on their way, bytes: none
+            for (int i = 0;; i ^= 1) {
+                const size_t o = next.fetch_add(1) * kChunk;
+                if (o < bytes) {
+                    if ((e = hipMemcpyAsync(two[i].p, (const char *)src + o, std::min(kChunk, bytes - o), hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+                    if ((e = hipEventRecord(two[i].ev, s)) != hipSuccess) return e;
+                    at[i] = o;
+                }
+                const size_t q = at[i ^ 1];
+                if (q < bytes) {
+                    if ((e = hipEventSynchronize(two[i ^ 1].ev)) != hipSuccess) return e;
+                    memcpy((char *)dst + q, two[i ^ 1].p, std::min(kChunk, bytes - q));
+                    at[i ^ 1] = bytes;
+                }
+                if (at[i] >= bytes) return e;
+            }
+        });
+    }
+
+private:
+    static constexpr size_t kChunk = 1 << 20, kMin = 8 * kChunk;
+    static constexpr int kThreads = 4;
+    struct Slot {
+        char *p = nullptr;
+        hipEvent_t ev = nullptr;
+    };
+    Slot slot_[2 * kThreads];
+    void *pin_ = nullptr;
+
+    bool staged(const void *host, size_t bytes)
+    {
+        if (bytes < kMin) return false;
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, host) != hipSuccess) (void)hipGetLastError();   // unknown to the runtime: pageable
+        else if (a.type != hipMemoryTypeUnregistered) return false;
+        if (!pin_) {
+            if (hipHostMalloc(&pin_, 2 * kThreads * kChunk, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                pin_ = nullptr;
+                return false;
+            }
+            for (int k = 0; k < 2 * kThreads; ++k) slot_[k].p = (char *)pin_ + k * kChunk;
+        }
+        for (Slot &t : slot_)
+            if (!t.ev) HU_CHECK(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+        return true;
+    }
+    template <class F>
+    void run(size_t bytes, F work)
+    {
+        int dev = 0;
+        HU_CHECK(hipGetDevice(&dev));
+        std::atomic<size_t> next{0};
+        hipError_t err[kThreads];
+        std::thread th[kThreads];
+        for (hipError_t &e : err) e = hipSuccess;
+        try {
+            for (int t = 1; t < kThreads; ++t)
+                th[t] = std::thread([&, t] {
+                    err[t] = hipSetDevice(dev);
+                    if (err[t] == hipSuccess) err[t] = work(slot_ + 2 * t, next);
+                });
+        } catch (const std::exception &) {   // no more threads: those that run, and this one, do it all
+        }
+        err[0] = work(slot_, next);
+        for (std::thread &t : th)
+            if (t.joinable()) t.join();
+        for (hipError_t e : err) HU_CHECK(e);
+    }
 };
 
 // Monotone mapping of doubles onto unsigned 64-bit integers so that min/max

@@ -191,3 +191,19 @@ def test_moving_window_poisson_matches_oracle(gpu, fp32, tol):
         if not err <= tol * scale:
             bad.append(name)
     assert not bad, bad
+
+
+@pytest.mark.parametrize("nx,ny", [(1024, 1023), (1024, 1024), (1031, 1025), (2000, 1100)])
+def test_large_arrays_travel_whole(gpu, nx, ny):
+    """Arrays of 8 MiB and more go through pinned buffers in chunks of 1 MiB by
+    several threads: just below and at that size, with a short last chunk, and
+    with more chunks than buffers.  Without a cycle the solve returns its guess
+    at unknown nodes and b at the others, bit for bit."""
+    cls = np.full((ny, nx), P.FIXED, np.uint8)
+    cls[1:-1, 1:-1] = P.UNKNOWN
+    rng = np.random.default_rng(nx * ny)
+    b, guess = rng.normal(size=(ny, nx)), rng.normal(size=(ny, nx))
+    for _ in range(2):
+        phi, cycles, _ = P.solve(1e-4, 1e-4, cls, b, phi0=guess, maxit=0)
+        assert cycles == 0
+        assert np.array_equal(phi, np.where(cls == P.UNKNOWN, guess, b))
