@@ -30,12 +30,11 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 # Algorithmic HBM bytes.  Per particle per push launch: the particle state
 # (int32 cell x/y, offset x/y, momentum x/y) read once and written once:
-# FP32 2*(8 + 16) = 48 B, FP64 2*(8 + 32) = 80 B.  Per cell per step: k_heh
-# reads Ex, Ey, Hz and the class byte and writes Ex', Hz'; k_ey reads Ey, Hz
-# and the class byte and writes Ey (currents only inside the bunch footprint):
-# FP32 13 + 8 + 9 + 4 = 34 B, FP64 25 + 16 + 17 + 8 = 66 B.
+# FP32 2*(8 + 16) = 48 B, FP64 2*(8 + 32) = 80 B.  Per cell per step k_sweep
+# reads Ex, Ey, Hz and the class byte and writes Ex', Ey', Hz' (currents only
+# inside the bunch footprint): FP32 13 + 12 = 25 B, FP64 25 + 24 = 49 B.
 B_PART = {True: 48, False: 80}
-B_CELL = {True: 34, False: 66}
+B_CELL = {True: 25, False: 49}
 
 
 def run_mw(cfg, fp32, steps, warmup, R, P, Q, stat):
