@@ -714,12 +714,23 @@ private:
     int dev_ = 0;
 };
 
+// Items and contributions are numbered, and sorted, in 32 bits: more than that
+// is refused, before any array is touched where the particle count shows it.
+void check_count(size_t count, int n)
+{
+    if (count > (size_t)INT_MAX)
+        throw Error(CSRST_EINVAL, hu::fmt("%d particles make %zu contributions; one call takes up to %d (deposit them in "
+                                          "several calls)", n, count, INT_MAX));
+}
+
 // A deposit: small ones by the node scan, large ones by the sort.  mode 0
 // writes the whole patch, mode 1 adds.  Returns the error bits.
 template <class Op>
 int deposit(const Op &op, int n, double *f, double div, int mode, hipStream_t st)
 {
+    constexpr bool kPack = Op::ITEMS == kMaxSeg;
     const size_t nodes = (size_t)op.p.nx * op.p.ny, items = (size_t)n * Op::ITEMS;
+    check_count(kPack ? items : items * Op::NN, n);
     if (node_scan_fits(items, nodes)) {
         const size_t wo = align256(items * sizeof(int2));
         const Lease ws(wo + items * Op::NN * sizeof(double), st);
@@ -742,7 +753,6 @@ int deposit(const Op &op, int n, double *f, double div, int mode, hipStream_t st
     }
     // currents use two of their four segments on average: count first, so that
     // only what there is is sorted
-    constexpr bool kPack = Op::ITEMS == kMaxSeg;
     const size_t so = align256(n);
     const Lease small(kPack ? so + (size_t)nb * sizeof(int) : 256, st);
     uint8_t *num = kPack ? (uint8_t *)small.base() : nullptr;
@@ -754,6 +764,7 @@ int deposit(const Op &op, int n, double *f, double div, int mode, hipStream_t st
         e = small.wait();
         cnt = (size_t)*(const volatile int *)small.total() * Op::NN;
         if (cnt == 0) return e;
+        check_count(cnt, n);
     }
     const size_t tmp = sort_tmp_bytes(cnt);
     const Lease ws(scratch_bytes(cnt, tmp), st);
@@ -935,6 +946,7 @@ int csrst_sf_current_density_noalloc(int order, int comp, double *J, int i0, int
         check_current_args(order, comp, dt, J, oldR, R, Q, n);
         const Patch p = make_patch(i0, j0, nx, ny, origin, dx);
         const size_t cnt = (size_t)n * slots_current(order), nodes = (size_t)nx * ny;
+        check_count(cnt, n);
         const size_t tmp = sort_tmp_bytes(cnt);      // a size query: nothing is allocated
         const size_t need = scratch_bytes(cnt, tmp);
         if (need > kScratchBytes)

@@ -235,7 +235,10 @@ int csrst_mw_poisson(csrst_mw *m, double tol, int maxit, int *cycles, double *re
  * node patches [ny][nx], x fastest.  `stream` is a hipStream_t (NULL: the
  * null stream); each call returns once its work has finished.  A stencil
  * that leaves the patch returns CSRST_EWINDOW (its values dropped or read as
- * zero); the other nodes are still written.
+ * zero); the other nodes are still written.  A deposit of more than 2^31 - 1
+ * contributions (particles times stencil nodes; for a current 4 times the
+ * particles, and the segments that there are times their nodes) returns
+ * CSRST_EINVAL.
  *
  * ScatterGatherImpl<IntOp,double>::gather / ::scatter
  * (ScatterGatherImpl.hh:27-64; IntCIC 70-194, IntS1 202-392, IntS2 407-641):
