@@ -436,8 +436,8 @@ template <int ORDER>
 __global__ void __launch_bounds__(kB) k_gather(Patch p, int lc, int s2bug, const double *f, const double *R, int n, double *out,
                          int *err)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
+    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;   // n may be 2^31 - 1
+    if (k >= (size_t)n) return;
     const vec2<double> od = pm::mk(1.0 / p.h[0], 1.0 / p.h[1]);
     const vec2<double> pp = pm::mk((R[2 * k] - p.o[0]) * od.x, (R[2 * k + 1] - p.o[1]) * od.y);
     bool bad = false;

@@ -7,11 +7,13 @@ every result is compared bit for bit.  The charge-density difference is
 checked against the discrete continuity equation with the GPU's own
 currents (dt div J = -(rho(R) - rho(oldR)) to round-off).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from csrst_amd import Commands, TwoGridStep, gaussian_bunch, shapefn as SF
-from csrst_amd._lib import CsrstError
+from csrst_amd._lib import CsrstError, check
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -185,3 +187,30 @@ def test_empty_bunch_and_one_node_patch(gpu):
     assert rho.shape == (2, 2) and same(rho, O.charge_density(0, (3, 2, 2, 2), org, dx, R, q))
     with pytest.raises(CsrstError):
         SF.getChargeDensity(0, (3, 2, 1, 1), org, dx, R, q)      # the stencil leaves a 1 x 1 patch
+
+
+def device_bytes(nbytes, fill):
+    """A device block of `nbytes` bytes of value `fill` (no host copy)."""
+    a = SF.DeviceArray(shape=(-(-nbytes // 8),))
+    assert SF.hip().hipMemset(a.ptr, C.c_int(fill), C.c_size_t(nbytes)) == 0
+    assert SF.hip().hipDeviceSynchronize() == 0
+    return a
+
+
+@pytest.mark.parametrize("order", [0, 2])
+def test_gather_beyond_2_30_particles(gpu, order):
+    """The coordinates of particle 2^30 and later lie past 2^31 doubles.  All
+    particles sit at the origin but the last three, one cell further."""
+    n = 2 ** 30 + 3
+    R, out = device_bytes(16 * n, 0), device_bytes(8 * n, 0xff)
+    last, head, tail = np.ones(6), np.empty(4), np.empty(8)
+    field = SF.DeviceArray(host=np.arange(64.0))
+    assert SF.hip().hipMemcpy(C.c_void_p(R.ptr.value + 16 * (n - 3)), last.ctypes.data_as(C.c_void_p), C.c_size_t(48), 1) == 0
+    rc = gpu.csrst_sg_gather(C.c_int(order), C.c_int(0), C.c_int(2), field.ptr, C.c_int(8), C.c_int(8), SF._v2((-4.25, -4.25)),
+                             SF._v2((1.0, 1.0)), R.ptr, C.c_int(n), out.ptr, None)
+    check(rc)
+    for a, at in ((head, 0), (tail, n - 8)):
+        assert SF.hip().hipMemcpy(a.ctypes.data_as(C.c_void_p), C.c_void_p(out.ptr.value + 8 * at), C.c_size_t(a.nbytes), 2) == 0
+    # splines reproduce a linear field: node (i, j) at (i + 1/2, j + 1/2) holds i + 8 j
+    want = np.where(np.arange(12) < 9, 3.75 * 9, 4.75 * 9)
+    assert np.abs(np.concatenate([head, tail]) - want).max() < 1e-13 * want.max()
