@@ -63,10 +63,14 @@ int slots_current(int order) { return kMaxSeg * (order == 0 ? 2 : order == 1 ? 6
 // that crosses more lines than one push can), and item(state, g, I, J, w): the
 // first node (relative to the patch) and the weights of item g, x fastest.
 
-__device__ __forceinline__ int rel(long long I, int i0)
+// first node I of a stencil relative to the patch's i0, or kOff if all its (at
+// most 4) nodes lie outside a patch of nx nodes.  Patches may have up to 2^31 - 1
+// nodes a side, so node indices past the first are formed as unsigned.
+constexpr int kOff = -8;
+__device__ __forceinline__ int rel(long long I, int i0, int nx)
 {
-    const long long d = I - i0, lim = 1 << 28;      // beyond any patch: a sum with a stencil's width stays an int
-    return (int)(d < -lim ? -lim : d > lim ? lim : d);
+    const long long d = I - i0;
+    return d < kOff || d >= nx ? kOff : (int)d;
 }
 
 // getCurrentDensityBase{X,Y} + getCurrentDensity{X,Y}: the trajectory oldR -> R
@@ -111,8 +115,8 @@ struct CurrentOp {
         const vec2<double> seg = pm::mk(b.x - a.x, b.y - a.y);
         pm::SegCurrent<double> sc;
         pm::segment_current(sc, ORDER, COMP, xi, xf, seg, s.covered, s.q, s.odt, s.delta);
-        I = rel(sc.I0, p.i0);
-        J = rel(sc.J0, p.j0);
+        I = rel(sc.I0, p.i0, p.nx);
+        J = rel(sc.J0, p.j0, p.ny);
 #pragma unroll
         for (int t = 0; t < NN; ++t) w[t] = sc.w[t];
     }
@@ -149,8 +153,8 @@ struct ChargeOp {
                 const double v = pm::charge_w<ORDER>(q, wx[a], wy[b]);
                 w[b * NX + a] = g == 0 ? v : -v;
             }
-        I = rel(I0, p.i0);
-        J = rel(J0, p.j0);
+        I = rel(I0, p.i0, p.nx);
+        J = rel(J0, p.j0, p.ny);
     }
 };
 
@@ -186,8 +190,8 @@ struct ScatterOp {
         for (int b = 0; b < NY; ++b)
 #pragma unroll
             for (int a = 0; a < NX; ++a) w[b * NX + a] = pm::scatter_w(st, a, b, v);
-        I = rel(st.I0, 0);      // the stencil is relative to the patch's node (0, 0)
-        J = rel(st.J0, 0);
+        I = rel(st.I0, 0, p.nx);      // the stencil is relative to the patch's node (0, 0)
+        J = rel(st.J0, 0, p.ny);
     }
 };
 
@@ -196,7 +200,7 @@ struct ScatterOp {
 template <class Op>
 __device__ __forceinline__ bool inside(const Op &op, int I, int J)
 {
-    return I >= 0 && J >= 0 && I + Op::NX <= op.p.nx && J + Op::NY <= op.p.ny;
+    return I >= 0 && J >= 0 && I <= op.p.nx - Op::NX && J <= op.p.ny - Op::NY;
 }
 
 // ---------------------------------------------------------------------------
@@ -415,9 +419,9 @@ __global__ void __launch_bounds__(64) k_emit(Op op, int n, const uint8_t *cnt, c
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < NN; ++t) {
-            const int i = I + t % Op::NX, j = J + t / Op::NX;
-            const bool in = on && i >= 0 && j >= 0 && i < op.p.nx && j < op.p.ny;
-            sk[tid * NN + t] = in ? (unsigned)j * (unsigned)op.p.nx + (unsigned)i : kEmpty;
+            const unsigned i = (unsigned)I + t % Op::NX, j = (unsigned)J + t / Op::NX;
+            const bool in = on && i < (unsigned)op.p.nx && j < (unsigned)op.p.ny;
+            sk[tid * NN + t] = in ? j * (unsigned)op.p.nx + i : kEmpty;
             sv[tid * NN + t] = in ? w[t] : 0.0;
         }
         __syncthreads();

@@ -214,3 +214,30 @@ def test_gather_beyond_2_30_particles(gpu, order):
     # splines reproduce a linear field: node (i, j) at (i + 1/2, j + 1/2) holds i + 8 j
     want = np.where(np.arange(12) < 9, 3.75 * 9, 4.75 * 9)
     assert np.abs(np.concatenate([head, tail]) - want).max() < 1e-13 * want.max()
+
+
+def test_charge_on_a_patch_wider_than_2_28(gpu):
+    """Columns past 2^28 = 268 435 456 of a patch of 3e8 x 2 nodes: the charge
+    lands on its own nodes, and one past the last column is reported."""
+    nx, ny, i0 = 300_000_000, 2, -1000
+    f = device_bytes(8 * nx * ny, 0xff)
+    R = SF.DeviceArray(host=np.array([[2.9e8 + 0.25 + i0, 0.5], [2.0e8 + 0.25 + i0, 0.5]]))
+    Q = SF.DeviceArray(host=np.array([1.0, 2.0]))
+
+    def node(i, j):
+        v = np.empty(1)
+        assert SF.hip().hipMemcpy(v.ctypes.data_as(C.c_void_p), C.c_void_p(f.ptr.value + 8 * (j * nx + i)), C.c_size_t(8), 2) == 0
+        return v[0]
+
+    def run():
+        return gpu.csrst_sf_charge_density(C.c_int(0), f.ptr, C.c_int(i0), C.c_int(0), C.c_int(nx), C.c_int(ny), SF._v2((0, 0)),
+                                           SF._v2((1, 1)), R.ptr, Q.ptr, C.c_int(2), None)
+
+    check(run())
+    for i, q in ((290_000_000, 1.0), (200_000_000, 2.0)):
+        assert [node(i + a, j) for j in (0, 1) for a in (0, 1)] == [0.375 * q, 0.125 * q] * 2
+    assert all(node(2 ** 28 + a, j) == 0 for j in (0, 1) for a in (-1, 0, 1))
+    # the second node of the stencil is past the patch: dropped and reported
+    R = SF.DeviceArray(host=np.array([[nx - 1 + 0.25 + i0, 0.5], [3.2e8, 0.5]]))
+    assert run() == -4
+    assert [node(nx - 1, j) for j in (0, 1)] == [0.375, 0.375] and node(0, 1) == 0 and node(2 ** 28, 0) == 0
