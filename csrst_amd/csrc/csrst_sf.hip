@@ -616,11 +616,13 @@ void reduce(const Scratch &s, size_t cnt, size_t nodes, double *f, double div, i
 // Workspaces of the calls.  hipMalloc and hipFree of a deposit's 200 MB took
 // 4 to 9 ms of a call whose kernels take 1 ms, so blocks are kept between
 // calls: a call leases one to itself and returns it after its stream has
-// finished.  Idle blocks are bounded to kKeep bytes per device, a block no call
-// has taken for kAge leases is freed, and all of them are freed before an
-// allocation is reported as failed.  Each has two words of pinned host memory
-// for the error flags (kernels store there, the host reads after the wait) and
-// one for a count.
+// finished.  A request takes a block of at most four times its size (and a few
+// MiB), so that a deposit's particle counts don't occupy its sort's workspace.
+// Idle blocks are bounded to kKeep bytes per device: a block larger than that is
+// freed at its return and leaves the others alone.  A block no call has taken
+// for kAge leases is freed, and all of them are freed before an allocation is
+// reported as failed.  Each has two words of pinned host memory for the error
+// flags (kernels store there, the host reads after the wait) and one for a count.
 class Lease {
 public:
     Lease(size_t bytes, hipStream_t st) : st_(st)
@@ -630,7 +632,9 @@ public:
         auto &v = idle();
         int best = -1;
         for (size_t q = 0; q < v.size(); ++q)
-            if (v[q].dev == dev_ && v[q].bytes >= bytes && (best < 0 || v[q].bytes < v[best].bytes)) best = (int)q;
+            if (v[q].dev == dev_ && v[q].bytes >= bytes && v[q].bytes <= 4 * bytes + kSmall &&
+                (best < 0 || v[q].bytes < v[best].bytes))
+                best = (int)q;
         if (best >= 0) {
             b_ = v[best];
             v.erase(v.begin() + best);
@@ -662,7 +666,16 @@ public:
         std::lock_guard<std::mutex> lock(mu());
         auto &v = idle();
         size_t kept = b_.bytes;
-        v.push_back(b_);
+        if (kept > kKeep) {
+            drop(b_);
+            return;
+        }
+        try {
+            v.push_back(b_);
+        } catch (const std::exception &) {     // no host memory to note it
+            drop(b_);
+            return;
+        }
         // newest first: what is beyond the bound or too long unused goes
         for (int q = (int)v.size() - 2; q >= 0; --q) {
             if (v[q].dev != dev_) continue;
@@ -672,10 +685,6 @@ public:
                 drop(v[q]);
                 v.erase(v.begin() + q);
             }
-        }
-        if (b_.bytes > kKeep) {
-            drop(v.back());
-            v.pop_back();
         }
     }
     unsigned char *base() const { return b_.p; }
@@ -696,7 +705,7 @@ private:
         int *host = nullptr;
         int dev = 0, age = 0;
     };
-    static constexpr size_t kKeep = (size_t)512 << 20;
+    static constexpr size_t kKeep = (size_t)512 << 20, kSmall = (size_t)4 << 20;
     static constexpr int kAge = 64;
     static std::mutex &mu()
     {

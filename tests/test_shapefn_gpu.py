@@ -241,3 +241,39 @@ def test_charge_on_a_patch_wider_than_2_28(gpu):
     R = SF.DeviceArray(host=np.array([[nx - 1 + 0.25 + i0, 0.5], [3.2e8, 0.5]]))
     assert run() == -4
     assert [node(nx - 1, j) for j in (0, 1)] == [0.375, 0.375] and node(0, 1) == 0 and node(2 ** 28, 0) == 0
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert SF.hip().hipDeviceSynchronize() == 0
+    assert SF.hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def sorted_deposit(n, comp=None):
+    """A charge (comp None) or current deposit of n S2 particles on a patch
+    large enough that it is sorted: 24 bytes of workspace a contribution, and
+    the sort's own."""
+    oldR = np.random.default_rng(n).uniform(6, 150, (n, 2))
+    if comp is None:
+        SF.getChargeDensity(2, (0, 0, 160, 160), (0.0, 0.0), (1.0, 1.0), oldR, np.ones(n))
+    else:
+        SF.getCurrentDensity(2, comp, (0, 0, 160, 160), (0.0, 0.0), (1.0, 1.0), 1.0, oldR, oldR + 0.25, np.ones(n))
+
+
+def test_kept_workspaces(gpu):
+    """Device memory that the deposits keep between calls: a request does not
+    take a block many times its size (the particle counts of a current deposit
+    would take the sort's, and the sort a second one), and a workspace beyond
+    the bound of 512 MiB is freed without the blocks that are idle."""
+    MiB = 2 ** 20
+    for _ in range(70):                         # blocks of other calls age out
+        sorted_deposit(30_000)
+    before = free_bytes()
+    sorted_deposit(600_000)                     # 230 MB and the sort's own
+    one = free_bytes()
+    assert 200 * MiB < before - one < 512 * MiB
+    sorted_deposit(400_000, comp=0)             # 1.5 segments of 12 contributions each: 170 MB and the sort's own
+    assert one - free_bytes() < 30 * MiB
+    sorted_deposit(2_000_000)                   # 770 MB and the sort's own
+    assert abs(one - free_bytes()) < 30 * MiB
