@@ -620,37 +620,23 @@ void reduce(const Scratch &s, size_t cnt, size_t nodes, double *f, double div, i
 // MiB), so that a deposit's particle counts don't occupy its sort's workspace.
 // Idle blocks are bounded to kKeep bytes per device: a block larger than that is
 // freed at its return and leaves the others alone.  A block no call has taken
-// for kAge leases is freed, and all of them are freed before an allocation is
-// reported as failed.  Each has two words of pinned host memory for the error
-// flags (kernels store there, the host reads after the wait) and one for a count.
+// for kAge leases is freed, and all of them are freed before any allocation of
+// this library is reported as failed.  Each has two words of pinned host memory
+// for the error flags (kernels store there, the host reads after the wait) and
+// one for a count.
 class Lease {
 public:
     Lease(size_t bytes, hipStream_t st) : st_(st)
     {
         HU_CHECK(hipGetDevice(&dev_));
-        std::lock_guard<std::mutex> lock(mu());
-        auto &v = idle();
-        int best = -1;
-        for (size_t q = 0; q < v.size(); ++q)
-            if (v[q].dev == dev_ && v[q].bytes >= bytes && v[q].bytes <= 4 * bytes + kSmall &&
-                (best < 0 || v[q].bytes < v[best].bytes))
-                best = (int)q;
-        if (best >= 0) {
-            b_ = v[best];
-            v.erase(v.begin() + best);
-        } else {
+        if (!take(bytes)) {
             b_.bytes = (bytes + (1 << 20) - 1) >> 20 << 20;
-            if (hipMalloc(&b_.p, b_.bytes) != hipSuccess) {
-                for (Block &x : v) drop(x);
-                v.clear();
-                if (hipMalloc(&b_.p, b_.bytes) != hipSuccess) {
-                    (void)hipGetLastError();
-                    throw Error(CSRST_ENOMEM, hu::fmt("hipMalloc of %zu bytes failed", b_.bytes));
-                }
-                (void)hipGetLastError();
-            }
+            hu::give_back().store(&Lease::drop_idle);
+            if (hu::device_alloc((void **)&b_.p, b_.bytes) != hipSuccess)
+                throw Error(CSRST_ENOMEM, hu::fmt("hipMalloc of %zu bytes failed", b_.bytes));
             b_.dev = dev_;
             if (hipHostMalloc(&b_.host, 64, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
                 (void)hipFree(b_.p);
                 throw Error(CSRST_ENOMEM, "hipHostMalloc failed");
             }
@@ -717,10 +703,31 @@ private:
         static std::vector<Block> *v = new std::vector<Block>;
         return *v;
     }
+    // the smallest idle block that serves `bytes`, if any
+    bool take(size_t bytes)
+    {
+        std::lock_guard<std::mutex> lock(mu());
+        auto &v = idle();
+        int best = -1;
+        for (size_t q = 0; q < v.size(); ++q)
+            if (v[q].dev == dev_ && v[q].bytes >= bytes && v[q].bytes <= 4 * bytes + kSmall &&
+                (best < 0 || v[q].bytes < v[best].bytes))
+                best = (int)q;
+        if (best < 0) return false;
+        b_ = v[best];
+        v.erase(v.begin() + best);
+        return true;
+    }
     static void drop(Block &x)
     {
         (void)hipFree(x.p);
         (void)hipHostFree(x.host);
+    }
+    static void drop_idle()
+    {
+        std::lock_guard<std::mutex> lock(mu());
+        for (Block &x : idle()) drop(x);
+        idle().clear();
     }
     Block b_;
     hipStream_t st_;

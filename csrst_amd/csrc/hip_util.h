@@ -49,6 +49,31 @@ inline std::string fmt(const char *f, ...)
     return buf;
 }
 
+// What frees the idle device memory that the library keeps between calls
+// (csrst_sf.hip's workspaces), if it keeps any.
+inline std::atomic<void (*)()> &give_back()
+{
+    static std::atomic<void (*)()> f{nullptr};
+    return f;
+}
+
+// hipMalloc that gives idle memory back before it fails, and leaves no error
+// for the next launch check to find.
+inline hipError_t device_alloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    void (*f)() = give_back().load();
+    if (e == hipErrorOutOfMemory && f) {
+        f();
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 // Owning device buffer.
 template <class T>
 struct DBuf {
@@ -69,10 +94,8 @@ struct DBuf {
         if (count == n && p) return;
         release();
         if (count == 0) return;
-        if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) {
-            p = nullptr;
+        if (device_alloc((void **)&p, count * sizeof(T)) != hipSuccess)
             throw Error(-2, fmt("hipMalloc of %zu bytes failed", count * sizeof(T)));
-        }
         n = count;
     }
     void zero(hipStream_t s) { if (n) HU_CHECK(hipMemsetAsync(p, 0, n * sizeof(T), s)); }

@@ -14,6 +14,7 @@ import pytest
 
 from csrst_amd import Commands, TwoGridStep, gaussian_bunch, shapefn as SF
 from csrst_amd._lib import CsrstError, check
+from csrst_amd.mw import MovingWindowStep
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -277,3 +278,24 @@ def test_kept_workspaces(gpu):
     assert one - free_bytes() < 30 * MiB
     sorted_deposit(2_000_000)                   # 770 MB and the sort's own
     assert abs(one - free_bytes()) < 30 * MiB
+
+
+def test_kept_workspaces_make_room(gpu):
+    """On a card with 1 GiB left besides a kept workspace of some 450 MB, a
+    window whose fields take 1.25 GiB still fits: the workspace is given back.
+    A window that does not fit at all is refused, and the next call works."""
+    sorted_deposit(800_000)
+    hold = []
+    try:
+        while free_bytes() > 2 ** 30 + 2 ** 26 and len(hold) < 8:      # memory freed late shows up here
+            hold.append(SF.DeviceArray(shape=((free_bytes() - 2 ** 30) // 8,)))
+        assert 2 ** 30 - 2 ** 26 < free_bytes() < 2 ** 30 + 2 ** 26
+        geom = dict(lenBefore=0.05, lenAfter=0.01, width=0.0128, phiDeg=10.0, ekinMeV=50.59, bz=0.1704)
+        MovingWindowStep(4096, 3150, 1e-5, 1e-5, order=1, fp32=False, **geom).close()
+        with pytest.raises(CsrstError) as e:
+            MovingWindowStep(16384, 8192, 1e-5, 1e-5, order=1, fp32=False, **geom)
+        assert e.value.code == -2
+        sorted_deposit(30_000)
+    finally:
+        for h in hold:
+            h.free()
