@@ -45,6 +45,15 @@ constexpr double kWeak = 0.03;
 
 int nblk(size_t n) { return (int)((n + kBlock - 1) / kBlock); }
 
+// kBlock rows j of a column i per workgroup, in a flat grid as the tiles are
+unsigned row_blocks(int nx, int ny) { return (unsigned)nx * (unsigned)nblk(ny); }
+__device__ __forceinline__ void row_block(int ny, int &i, int &j)
+{
+    const unsigned per = (unsigned)(ny + kBlock - 1) / kBlock;
+    i = (int)(blockIdx.x / per);
+    j = (int)(blockIdx.x % per) * kBlock + (int)threadIdx.x;
+}
+
 // ---------------------------------------------------------------------------
 // set-up
 
@@ -52,7 +61,9 @@ int nblk(size_t n) { return (int)((n + kBlock - 1) / kBlock); }
 __global__ void __launch_bounds__(kBlock) k_act(const uint8_t *cls, uint8_t *act, int nx, int ny, int pitch, int M)
 {
     __shared__ uint8_t t[kTile][kTile + 4];
-    const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile, a = threadIdx.x % kTile, b = threadIdx.x / kTile;
+    const int a = threadIdx.x % kTile, b = threadIdx.x / kTile;
+    int i0, j0;
+    tile_origin(nx, i0, j0);
     for (int r = b; r < kTile; r += kBlock / kTile) {
         const int i = i0 + a, j = j0 + r;
         t[r][a] = i < nx && j < ny && cls[(size_t)j * nx + i] == kUnknown ? 1 : 0;
@@ -523,7 +534,8 @@ __device__ __forceinline__ double residual_at(const Level &L, int i, int j)
 // restriction for long lines, a thread per coarse node
 __global__ void __launch_bounds__(kBlock) k_restrict_long(Level F, Level C)
 {
-    const int j = blockIdx.x * kBlock + threadIdx.x, I = blockIdx.y;
+    int I, j;
+    row_block(C.ny, I, j);
     if (j >= C.ny) return;
     const int p = row_pos(j, F.lane);
     double v = 0.0;
@@ -587,7 +599,8 @@ __global__ void __launch_bounds__(kBlock) k_residual(Level L, double *partial)
 }
 __global__ void __launch_bounds__(kBlock) k_residual_long(Level L, double *partial)
 {
-    const int j = blockIdx.x * kBlock + threadIdx.x, i = blockIdx.y;
+    int i, j;
+    row_block(L.ny, i, j);
     double s = 0.0;
     if (j < L.ny) {
         const size_t k = L.at(i, j);
@@ -595,7 +608,7 @@ __global__ void __launch_bounds__(kBlock) k_residual_long(Level L, double *parti
         L.res[k] = s;
     }
     s = block_sum(s * s);
-    if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = s;
+    if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
 __global__ void __launch_bounds__(kBlock) k_sum_final(const double *partial, int nb, double *out)
@@ -615,7 +628,9 @@ __global__ void __launch_bounds__(kBlock) k_load(const uint8_t *cls, const doubl
                                                  double *partial)
 {
     __shared__ double tr[kTile][kTile + 1], tp[kTile][kTile + 1];
-    const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile, a = threadIdx.x % kTile, row = threadIdx.x / kTile;
+    const int a = threadIdx.x % kTile, row = threadIdx.x / kTile;
+    int i0, j0;
+    tile_origin(L.nx, i0, j0);
     double s = 0.0;
     for (int r = row; r < kTile; r += kBlock / kTile) {
         const int i = i0 + a, j = j0 + r;
@@ -645,14 +660,16 @@ __global__ void __launch_bounds__(kBlock) k_load(const uint8_t *cls, const doubl
         }
     }
     s = block_sum(s);
-    if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = s;
+    if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
 // Solution out: unknowns from the level, identity rows phi = b.
 __global__ void __launch_bounds__(kBlock) k_store(const uint8_t *cls, const double *b, Level L, double *phi)
 {
     __shared__ double t[kTile][kTile + 1];
-    const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile, a = threadIdx.x % kTile, row = threadIdx.x / kTile;
+    const int a = threadIdx.x % kTile, row = threadIdx.x / kTile;
+    int i0, j0;
+    tile_origin(L.nx, i0, j0);
     for (int r = row; r < kTile; r += kBlock / kTile) {
         const int i = i0 + r, j = j0 + a;
         t[r][a] = i < L.nx && j < L.ny ? L.phi[L.at(i, j)] : 0.0;
@@ -706,7 +723,7 @@ void half_sweep(const Level &L, const Level &C, int color, hipStream_t s)
 void restrict_to(const Level &F, const Level &C, hipStream_t s)
 {
     if (is_long(F)) {
-        k_restrict_long<<<dim3((C.ny + kBlock - 1) / kBlock, C.nx), kBlock, 0, s>>>(F, C);
+        k_restrict_long<<<row_blocks(C.nx, C.ny), kBlock, 0, s>>>(F, C);
         k_smooth_long<kZero><<<((C.nx + 1) / 2 + kWaves - 1) / kWaves, kBlock, 0, s>>>(C, C, 0);
     } else {
         const int nb = (C.nx + kWaves - 1) / kWaves;
@@ -760,7 +777,7 @@ void Solver::setup(int nx, int ny, double hx, double hy, const uint8_t *cls, hip
     cols_.alloc(align(m0) + nx * sizeof(ColRows));
     uint8_t *act = cols_.p;
     ColRows *rows = reinterpret_cast<ColRows *>(cols_.p + align(m0));
-    k_act<<<dim3((nx + kTile - 1) / kTile, (pitch + kTile - 1) / kTile), kBlock, 0, s_>>>(cls, act, nx, ny, pitch, M);
+    k_act<<<num_tiles(nx, pitch), kBlock, 0, s_>>>(cls, act, nx, ny, pitch, M);
     k_rows<<<(nx + kWaves - 1) / kWaves, kBlock, 0, s_>>>(act, rows, nx, ny, pitch, M);
     HU_LAUNCH_CHECK();
     // the first kMaxTab run starts get tables (a straight chamber has one)
@@ -782,8 +799,7 @@ void Solver::setup(int nx, int ny, double hx, double hy, const uint8_t *cls, hip
     // level-0 residual
     size_t off = 0, cells = 0;
     auto take = [&](size_t b) { const size_t o = off; off += align(b); return o; };
-    const size_t tiles = (size_t)((nx + kTile - 1) / kTile) * ((pitch + kTile - 1) / kTile);
-    const size_t parts = std::max(tiles, (size_t)((ny + kBlock - 1) / kBlock) * nx);
+    const size_t parts = std::max(num_tiles(nx, pitch), row_blocks(nx, ny));
     const size_t oStart = take((size_t)nt * sizeof(int)), oTail = take(sizeof(Tail)), oPart = take(parts * sizeof(double));
     const size_t oG = take((size_t)nl * ny * sizeof(double)), oGt = take((size_t)nl * nt * pitch * sizeof(double));
     for (const Level &L : lv_) cells += (size_t)L.nx * pitch;
@@ -870,9 +886,8 @@ double Solver::resnorm()
 {
     const Level &L = lv_[0];
     if (is_long(L)) {
-        const dim3 grid((L.ny + kBlock - 1) / kBlock, L.nx);
-        npart_ = (int)(grid.x * grid.y);
-        k_residual_long<<<grid, kBlock, 0, s_>>>(L, partial_);
+        npart_ = (int)row_blocks(L.nx, L.ny);
+        k_residual_long<<<npart_, kBlock, 0, s_>>>(L, partial_);
     } else {
         npart_ = (L.nx + kWaves - 1) / kWaves;
         with_rows(L, [&](auto m) { k_residual<decltype(m)::value><<<npart_, kBlock, 0, s_>>>(L, partial_); });
@@ -883,9 +898,8 @@ double Solver::resnorm()
 double Solver::begin(const double *b, const double *phi0)
 {
     const Level &L = lv_[0];
-    const dim3 grid((L.nx + kTile - 1) / kTile, (L.pitch + kTile - 1) / kTile);
-    npart_ = (int)(grid.x * grid.y);
-    k_load<<<grid, kBlock, 0, s_>>>(cls_, b, phi0, L, partial_);
+    npart_ = (int)num_tiles(L.nx, L.pitch);
+    k_load<<<npart_, kBlock, 0, s_>>>(cls_, b, phi0, L, partial_);
     return read_norm();
 }
 
@@ -898,7 +912,7 @@ double Solver::residual(const double *b, const double *phi)
 void Solver::store(const double *b, double *phi)
 {
     const Level &L = lv_[0];
-    k_store<<<dim3((L.nx + kTile - 1) / kTile, (L.ny + kTile - 1) / kTile), kBlock, 0, s_>>>(cls_, b, L, phi);
+    k_store<<<num_tiles(L.nx, L.ny), kBlock, 0, s_>>>(cls_, b, L, phi);
     HU_LAUNCH_CHECK();
 }
 

@@ -1366,7 +1366,9 @@ template <class Get, class Put>
 __device__ __forceinline__ void level_to_image(const pmg::Level &L, Get get, Put put)
 {
     __shared__ float t[kT][kT + 1];
-    const int i0 = blockIdx.x * kT, j0 = blockIdx.y * kT, a = threadIdx.x % kT, row = threadIdx.x / kT;
+    const int a = threadIdx.x % kT, row = threadIdx.x / kT;
+    int i0, j0;
+    pmg::tile_origin(L.nx, i0, j0);
     for (int r = row; r < kT; r += kB / kT) {
         const int i = i0 + r, j = j0 + a;
         const size_t k = L.at(i, j);
@@ -1395,7 +1397,9 @@ __global__ void __launch_bounds__(kB) k_err_tgt(pmg::Level L, const double *psta
 __global__ void __launch_bounds__(kB) k_dir_in(pmg::Level L, const float *img, float *c)
 {
     __shared__ float t[kT][kT + 1];
-    const int i0 = blockIdx.x * kT, j0 = blockIdx.y * kT, a = threadIdx.x % kT, row = threadIdx.x / kT;
+    const int a = threadIdx.x % kT, row = threadIdx.x / kT;
+    int i0, j0;
+    pmg::tile_origin(L.nx, i0, j0);
     for (int r = row; r < kT; r += kB / kT) {
         const int i = i0 + a, j = j0 + r;
         t[r][a] = i < L.nx && j < L.ny ? img[(size_t)j * L.nx + i] : 0.f;
@@ -1407,7 +1411,7 @@ __global__ void __launch_bounds__(kB) k_dir_in(pmg::Level L, const float *img, f
     }
 }
 
-dim3 tile_grid(const pmg::Level &L) { return dim3((L.nx + kT - 1) / kT, (L.pitch + kT - 1) / kT); }
+unsigned tile_grid(const pmg::Level &L) { return pmg::num_tiles(L.nx, L.pitch); }
 
 // c . A c's row k: the level's 5-point operator with the unknowns' couplings
 // only, as the multigrid applies it

@@ -125,7 +125,18 @@ private:
 // workgroup's 32 x 32 tile with its origin at column i0, row j0.  Callers
 // read the image with x across the lanes, keep the tile in LDS, and write the
 // level with y across the lanes (or the reverse); the odd LDS pitch keeps both
-// passes free of bank conflicts.
+// passes free of bank conflicts.  The tiles are a flat grid: a grid's y dimension
+// ends at 65535, and a grid may have more columns, or rows of tiles, than that.
 constexpr int kTile = 32;
+inline unsigned num_tiles(int nx, int rows)
+{
+    return (unsigned)((nx + kTile - 1) / kTile) * (unsigned)((rows + kTile - 1) / kTile);
+}
+__device__ __forceinline__ void tile_origin(int nx, int &i0, int &j0)
+{
+    const unsigned across = (unsigned)(nx + kTile - 1) / kTile;
+    i0 = (int)(blockIdx.x % across) * kTile;
+    j0 = (int)(blockIdx.x / across) * kTile;
+}
 
 }  // namespace pmg

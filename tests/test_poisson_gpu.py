@@ -207,3 +207,39 @@ def test_large_arrays_travel_whole(gpu, nx, ny):
         phi, cycles, _ = P.solve(1e-4, 1e-4, cls, b, phi0=guess, maxit=0)
         assert cycles == 0
         assert np.array_equal(phi, np.where(cls == P.UNKNOWN, guess, b))
+
+
+def test_more_columns_than_a_grid_dimension(gpu):
+    """131100 columns of 2049 rows: more, also on the first coarse level, than
+    the 65535 workgroups of a grid's y dimension.  The unknowns are a strip
+    near the end, so that the oracle solves the strip alone."""
+    nx, ny, x0, w = 131100, 2049, 131008, 40
+    small = np.zeros((ny, 128), np.uint8)               # the strip with the same columns on each of six levels
+    small[1:-1, 64:64 + w] = 1
+    bs = np.where(small, np.random.default_rng(5).normal(size=small.shape) + 1.0, 0.0)
+    ref = O.poisson_solve(2e-4, 1e-4, small, small, bs)[:, 64:64 + w]
+    cls = np.full((ny, nx), P.FIXED, np.uint8)
+    cls[1:-1, x0:x0 + w] = P.UNKNOWN
+    b = np.zeros((ny, nx))
+    b[:, x0:x0 + w] = bs[:, 64:64 + w]
+    phi, cyc, res = P.solve(2e-4, 1e-4, cls, b, tol=1e-12, maxit=200)
+    err = np.abs(phi[:, x0:x0 + w] - ref).max() / np.abs(ref).max()
+    print("%d x %d: %d cycles, residual %.1e, error %.1e" % (nx, ny, cyc, res, err))
+    assert res <= 1e-12 and err <= 1e-9
+    assert not phi[:, :x0].any() and not phi[:, x0 + w:].any()
+
+
+def test_more_rows_than_a_grid_dimension_of_tiles(gpu):
+    """Two columns of 2.1e6 unknowns: more than 65535 tiles of 32 rows, and
+    2051 chunks of a line.  The solution is chosen and the right-hand side made
+    from it; the x couplings keep the operator's condition under 10."""
+    ny = 2_100_001
+    sol = np.zeros((ny, 4))
+    sol[1:-1, 1:3] = np.random.default_rng(6).normal(size=(ny - 2, 2))
+    b = np.zeros((ny, 4))
+    b[1:-1, 1:3] = 4 * sol[1:-1, 1:3] - sol[:-2, 1:3] - sol[2:, 1:3] - sol[1:-1, 0:2] - sol[1:-1, 2:4]
+    cls = np.full((ny, 4), P.FIXED, np.uint8)
+    cls[1:-1, 1:3] = P.UNKNOWN
+    phi, cyc, res = P.solve(1.0, 1.0, cls, b, tol=1e-12, maxit=100)
+    print("4 x %d: %d cycles, residual %.1e, error %.1e" % (ny, cyc, res, np.abs(phi - sol).max()))
+    assert res <= 1e-12 and np.abs(phi - sol).max() <= 1e-10
