@@ -5,6 +5,8 @@
 - FP32 split precision against FP64 on a moving bunch (fields and wake);
 - window motion keeps the bunch inside and positions advance at ~c.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -243,3 +245,28 @@ def test_field_step_edges(gpu, W, H, pml):
         for name, a, b in (("Ex", got[0], ex), ("Ey", got[1], ey), ("Hz", got[2] + got[3], hz)):
             err = np.abs(a - b).max() / np.abs(b).max()
             assert err < tol, (name, fp32, err)
+
+
+@pytest.mark.parametrize("W,H,n,fp32", [(512, 100, 20_000, True), (512, 100, 0, False), (4096, 1024, 200_000, True)])
+def test_step_times_add_up(gpu, W, H, n, fp32):
+    """The device-clock times of a call (push, sweeps, moves, sort) are taken
+    from one kernel's start to the next one's: each is non-negative, call by
+    call, and a call's sum is most of the wall time of its steps and no more."""
+    b = O.Bend(Nx=NX, Ny=NY, **GEOM)
+    hx, hy = (v / (W // 512) for v in b.hr)
+    m = MovingWindowStep(W, H, hx, hy, order=1, fp32=fp32, sortEvery=7, statModulus=5, pml=16, **GEOM)
+    if n:
+        m.init_bunch(*gaussian_bunch(n, (0.03, 0.0064), 0.2e-3, 0.1e-3, 100.0, 1.0, seed=3, energy_spread=1e-3))
+    else:
+        m.place(0, 0)
+    m.step(20)
+    for steps in [1] * 40 + [200] * 3:
+        t0 = time.perf_counter()
+        m.step(steps)
+        wall = 1e3 * (time.perf_counter() - t0) / steps
+        t = m.timing()
+        assert all(v >= 0 for v in t.values()), t
+        assert (t["push_ms"] > 0) == (n > 0) and t["sweep_ms"] > 0
+        assert sum(t.values()) <= wall, (t, wall)
+        if steps > 1:
+            assert sum(t.values()) >= 0.5 * wall, (t, wall)
