@@ -573,21 +573,41 @@ __device__ __forceinline__ void rotate_in(T (&o)[N], T v)
     o[N - 1] = v;
 }
 
-// Up to this many particles a thread takes one particle (PPT = 1) and adds its
-// segments straight into the LDS tile; above, it takes a run.  The run form
-// needs 1024 particles per workgroup and ends with passes per distinct anchor,
-// so it takes 57 to 120 us however few there are; the other form's LDS atomics
-// collide on a dense bunch and cost 0.16 us per 1000 particles.  us per push,
-// bunch of 20 x 10 cells in the bend, one particle / run:
-//   FP32 S1  1e5 17/58, 7e5 64/63    S2  1e5 31/80, 3e5 73/85, 7e5 143/87
-//   FP32 S0  1e5 12/58, 1.5e6 72/78  FP64 S2  2e4 20/115, 7e5 105/141, 1.5e6 209/180
+// Up to this many particles a thread takes one particle (PPT = 1): lanes of a
+// quad that share an anchor add their segments in registers, and each sum goes
+// straight into the LDS tile.  Above, a thread takes a run: that form needs 1024
+// particles per workgroup and ends with passes per distinct anchor, so it takes
+// 20 to 110 us however few there are, and less per particle.  us per push, one
+// particle / run, sigma 20 x 10 | 1.5 x 1.5 cells at 3 degrees:
+//   FP32 S0  1e5  7/46 |  7/18   3.4e5 14/47 | 12/18   1.4e6 37/64 | 34/34
+//        S1  1e5 10/55 | 11/22   3.4e5 28/56 | 19/23   6.4e5 39/59 | 28/27
+//        S2  1e5 15/67 | 16/25   3.4e5 49/67 | 27/26
+//   FP64 S0  1e5  8/52 |  8/20   4.9e5 20/55 | 24/23   1.0e6 35/73
+//        S1  1e5 11/68 | 10/25   4.9e5 29/72 | 32/31   1.0e6 50/103
+//        S2  1e5 16/91 | 13/32   4.9e5 41/95 | 40/37   1.0e6 69/133
+// so a dense FP64 bunch changes over at half the count.
+//
+// The tile of this form is FP64 whatever T is (ds_add_f64), so that in FP32 only
+// the additions to the global plane round, one per node and workgroup.  A dense
+// bunch has many workgroups on a node; its workgroups are as many particles as
+// the run form's.  L2 error of FP32 Jx of sorted particles against FP64, one
+// particle / run:
+//   80 per cell  (256 a workgroup)   S0 4.5e-8/5.2e-8  S1 5.3e-8/6.2e-8  S2 6.5e-8/7.1e-8
+//   199 per cell (256)               S0 5.1e-8/5.7e-8  S1 6.5e-8/6.8e-8  S2 6.4e-8/6.4e-8
+//   517 per cell (1024)              S0 5.2e-8/6.2e-8  S1 5.9e-8/6.8e-8  S2 8.0e-8/8.8e-8
+// (256 at 517 per cell: S1 7.7e-8, S2 1.0e-7; with an FP32 tile 256 at 80 per
+// cell: S1 1.2e-7, S2 1.5e-7).  Particles that were never sorted fall outside a
+// workgroup's tile one by one, where the run form adds four first (S2 3.4e-7 /
+// 2.1e-7): in FP32 they take the run form.
 template <class T>
 constexpr int few_particles(int order)
 {
     return sizeof(T) == 8 ? 1000000 : order == 0 ? 1500000 : order == 1 ? 650000 : 350000;
 }
+constexpr int kDense = 200, kDenseWG = 1024;              // FP32: particles per cell, particles per workgroup beyond
+constexpr int kDense64 = 15000, kFewDense64 = 500000;     // FP64: particles per cell, few_particles beyond
 
-// Push of one workgroup chunk (kB PPT sorted particles): thread t owns
+// Push of one workgroup chunk (NB PPT sorted particles): thread t owns
 // particles base + PPT t .. + PPT - 1, so its consecutive particles share a
 // cell and their segment currents share stencil anchors.  Currents collect in
 // kSlots register slots per lane (one anchor each).  A segment whose anchor
@@ -604,14 +624,15 @@ constexpr int few_particles(int order)
 // (c3 at 1-10 deg: the cooperative form 13-25 % faster; c2 at 1-8 deg: 2-8 %
 // slower; along x the cooperative path in the loop costs 20 %), so the step
 // times the two against each other and keeps the faster (csrst_mw_step).
-template <class T, int ORDER, int COMP, bool MISSCOOP, int PPT>
-__global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3))) k_push(Parts<T> p, Fields<T> f, Geo g, PushConst<T> c, WinState *ws)
+template <class T, int ORDER, int COMP, bool MISSCOOP, int PPT, int NB>
+__global__ void __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(1, NB > 768 ? 4 : 3))) k_push(Parts<T> p, Fields<T> f, Geo g, PushConst<T> c, WinState *ws)
 {
     tick(ws, COMP == 0 ? kPush0 : kPush1);
-    __shared__ T acc[kTH * kTW];
+    using A = std::conditional_t<PPT == 1, double, T>;
+    __shared__ A acc[kTH * kTW];
     __shared__ int pbox[4];          // particle cell box of the chunk (min x, min y, -max x, -max y)
     const int tid = threadIdx.x, lane = tid & 63;
-    const int base = blockIdx.x * (kB * PPT);
+    const int base = blockIdx.x * (NB * PPT);
     const int kt = base + tid * PPT;            // this thread's first particle
     const int wx0 = ws->wx0, wy0 = ws->wy0, rx = ws->rx, ry = ws->ry;
     const vec2<T> p0 = pm::mk((T)ws->p0[0], (T)ws->p0[1]);
@@ -625,7 +646,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
     if (tid == 0) {
         pbox[0] = INT_MAX; pbox[1] = INT_MAX; pbox[2] = INT_MAX; pbox[3] = INT_MAX;
     }
-    for (int q = tid; q < kTH * kTW; q += kB) acc[q] = T(0);
+    for (int q = tid; q < kTH * kTW; q += NB) acc[q] = A(0);
     __syncthreads();
     int err = 0;
     int bminx = INT_MAX, bminy = INT_MAX, bmaxx = INT_MIN, bmaxy = INT_MIN;
@@ -638,7 +659,8 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
     auto node_add = [&](int gxn, int gyn, T v) {
         const int li = gxn - ax, lj = gyn - ay;
         if (li >= 0 && li < kTW && lj >= 0 && lj < kTH) {
-            atomicAdd(&acc[lj * kTW + li], v);
+            if constexpr (PPT == 1) unsafeAtomicAdd(&acc[lj * kTW + li], (A)v);   // ds_add_f64
+            else atomicAdd(&acc[lj * kTW + li], v);
         } else {
             const int i = gxn - wx0, j = gyn - wy0;
             if (i < 0 || i > W - 1 || j < 0 || j > H - 1) err |= 1;
@@ -879,7 +901,6 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
             const vec2<T> delta = pm::mk(e.x - o.x, e.y - o.y);
             const int nseg = live ? xs.n - 1 : 0;
             if constexpr (PPT == 1) {
-                // every segment straight into the LDS tile
 #pragma unroll 1
                 for (int s = 0; s < 3; ++s) {
                     const bool act = s < nseg;
@@ -889,7 +910,17 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
                     const vec2<T> xf = sel(s == 0, xs.s[1], sel(s == 1, xs.s[2], xs.s[3]));
                     const T tau = s == 0 ? xs.f[1] - xs.f[0] : s == 1 ? xs.f[2] - xs.f[1] : xs.f[3] - xs.f[2];
                     seg_current(sc, xi, xf, tau, delta, gx0, gy0);
-                    if (act) lane_add(sc.I0, sc.J0, sc.w);
+                    // one add per quad whose lanes share an anchor, else one per lane
+                    const int aI = sc.I0, aJ = act ? sc.J0 : INT_MIN + lane;
+                    const bool one = aI == dpp_i<0xb1, 0xf>(0, aI) && aJ == dpp_i<0xb1, 0xf>(0, aJ) &&
+                                     aI == dpp_i<0x4e, 0xf>(0, aI) && aJ == dpp_i<0x4e, 0xf>(0, aJ) &&
+                                     aI == dpp_i<0x1b, 0xf>(0, aI) && aJ == dpp_i<0x1b, 0xf>(0, aJ);
+#pragma unroll
+                    for (int t = 0; t < NN; ++t) {
+                        const T q = quad_sum(sc.w[t]);
+                        sc.w[t] = one ? q : sc.w[t];
+                    }
+                    if (act && (!one || (lane & 3) == 0)) lane_add(sc.I0, sc.J0, sc.w);
                 }
             } else {
             // third segments (a push crossing a cell column and a cell row) are
@@ -1011,8 +1042,8 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(1, 3)))
         atomicMin(&b[0], pbox[0]); atomicMin(&b[1], pbox[1]);
         atomicMin(&b[2], pbox[2]); atomicMin(&b[3], pbox[3]);
     }
-    for (int q = tid; q < kTH * kTW; q += kB) {
-        const T v = acc[q];
+    for (int q = tid; q < kTH * kTW; q += NB) {
+        const T v = (T)acc[q];
         if (v == T(0)) continue;
         const int i = ax + (q % kTW) - wx0, j = ay + (q / kTW) - wy0;
         if (i < 0 || i > W - 1 || j < 0 || j > H - 1) { atomicOr(&ws->err, 1); continue; }
@@ -1887,6 +1918,15 @@ struct csrst_mw {
     // the push sends slot misses through the wavefront (MISSCOOP).  Chosen by
     // timing: every kRetune steps one step runs each form and the faster stays
     bool tilted = false;
+    // the push takes one particle per thread (few_particles)
+    double perCell = 0;           // density of the bunch at its start: particles per cell
+    bool isSorted = false;        // the particles have been sorted since
+    bool few() const
+    {
+        if (f32) return n <= mw::few_particles<float>(p.order);
+        return n <= (perCell > mw::kDense64 ? mw::kFewDense64 : mw::few_particles<double>(p.order));
+    }
+    bool one_particle() const { return few() && (isSorted || !f32); }
     int tunePhase = 0;            // 0 idle, 1 timing the cooperative form, 2 the per-lane form
     int nextTune = 0;             // step at which the next comparison starts
     float tuneMs = 0;             // push time of the cooperative form
@@ -1983,14 +2023,16 @@ void launch_push(csrst_mw *m)
 {
     mw::PushConst<T> c;
     push_consts(m, c);
-    auto go = [&](auto kern, int ppt) {
-        const int chunk = mw::kB * ppt;
-        hipLaunchKernelGGL(kern, dim3((m->n + chunk - 1) / chunk), dim3(mw::kB), 0, m->s, m->parts<T>(m->partBuf),
+    constexpr int PPT = mw::kPPT, kB = mw::kB, kBig = sizeof(T) == 4 ? mw::kDenseWG : kB;
+    auto go = [&](auto kern, int ppt, int nt) {
+        const int chunk = nt * ppt;
+        hipLaunchKernelGGL(kern, dim3((m->n + chunk - 1) / chunk), dim3(nt), 0, m->s, m->parts<T>(m->partBuf),
                            m->fields<T>(), m->geo, c, m->ws.p);
     };
-    if (m->n <= mw::few_particles<T>(ORDER)) go(mw::k_push<T, ORDER, COMP, false, 1>, 1);
-    else if (m->tilted) go(mw::k_push<T, ORDER, COMP, true, mw::kPPT>, mw::kPPT);
-    else go(mw::k_push<T, ORDER, COMP, false, mw::kPPT>, mw::kPPT);
+    if (m->one_particle() && m->perCell <= mw::kDense) go(mw::k_push<T, ORDER, COMP, false, 1, kB>, 1, kB);
+    else if (m->one_particle()) go(mw::k_push<T, ORDER, COMP, false, 1, kBig>, 1, kBig);
+    else if (m->tilted) go(mw::k_push<T, ORDER, COMP, true, PPT, kB>, PPT, kB);
+    else go(mw::k_push<T, ORDER, COMP, false, PPT, kB>, PPT, kB);
 }
 
 template <class T, int COMP>
@@ -2005,6 +2047,7 @@ void push_dispatch(csrst_mw *m)
 template <class T>
 void sort_particles(csrst_mw *m)
 {
+    m->isSorted = true;
     const int nb = (m->n + mw::kB - 1) / mw::kB;
     int *boxPart = reinterpret_cast<int *>(m->partial.p);   // kRedBlocks x 4 ints
     mw::k_box_partial<T><<<mw::kRedBlocks, mw::kB, 0, m->s>>>(m->parts<T>(m->partBuf), boxPart, m->ws.p);
@@ -2297,6 +2340,20 @@ int csrst_mw_init_bunch(csrst_mw *m, const double *R, const double *P, const dou
         for (int k = 0; k < n; ++k) { sp[0] += P[2 * k]; sp[1] += P[2 * k + 1]; }
         double p0[2] = {(double)(sp[0] / n), (double)(sp[1] / n)};
         if (f32) { p0[0] = (double)(float)p0[0]; p0[1] = (double)(float)p0[1]; }
+        // density at the centre of a Gaussian of the positions' covariance (in cells)
+        m->perCell = 0;
+        if (n <= (f32 ? mw::few_particles<float>(m->p.order) : mw::few_particles<double>(m->p.order))) {
+            double mean[2] = {0, 0}, cov[3] = {0, 0, 0};
+            const double ihx = 1 / m->geo.h[0], ihy = 1 / m->geo.h[1];
+            for (int k = 0; k < n; ++k) {
+                const double x = (R[2 * k] - R[0]) * ihx, y = (R[2 * k + 1] - R[1]) * ihy;
+                mean[0] += x; mean[1] += y;
+                cov[0] += x * x; cov[1] += x * y; cov[2] += y * y;
+            }
+            const double c0 = cov[0] - mean[0] * mean[0] / n, c1 = cov[1] - mean[0] * mean[1] / n,
+                         c2 = cov[2] - mean[1] * mean[1] / n;
+            m->perCell = n / std::max(1.0, 2 * M_PI * sqrt(std::max(0.0, c0 * c2 - c1 * c1)) / n);
+        }
         for (int k = 0; k < n; ++k) {
             const double ux = (R[2 * k] - m->geo.org[0]) / m->geo.h[0];
             const double uy = (R[2 * k + 1] - m->geo.org[1]) / m->geo.h[1];
@@ -2327,6 +2384,7 @@ int csrst_mw_init_bunch(csrst_mw *m, const double *R, const double *P, const dou
         HU_CHECK(hipMemcpy(m->partBuf.p, host.data(), host.size(), hipMemcpyHostToDevice));
         mw::k_state_init<<<1, 1, 0, m->s>>>(m->ws.p, wx0, wy0);
         mw::k_set_p0<<<1, 1, 0, m->s>>>(m->ws.p, p0[0], p0[1]);
+        m->isSorted = false;
         m->tilted = false;
         m->tunePhase = 0;
         m->nextTune = 0;
@@ -2398,7 +2456,7 @@ int csrst_mw_step(csrst_mw *m, int nsteps)
             HU_CHECK(hipEventElapsedTime(&b, m->ev[2], m->ev[3]));
             return a + b;
         };
-        const bool two = m->n > (m->f32 ? mw::few_particles<float>(m->p.order) : mw::few_particles<double>(m->p.order));
+        const bool two = m->n > 0 && !(m->few() && (!m->f32 || m->p.sortEvery > 0));   // the first step sorts
         for (int k = 0; k < nsteps; ++k) {
             bool trial = false;
             if (two && m->tunePhase == 0 && m->steps >= m->nextTune) {

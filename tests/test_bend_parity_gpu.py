@@ -276,6 +276,76 @@ def test_push_forms_vs_oracle(gpu, fp32, n, order):
     assert all(e < t for e, t in zip(err, tol)), err
 
 
+def sorted_push(order, fp32, n, sigma, comp, seed, tilt=0.0):
+    """One push of n particles, sorted as a run's are, on uniform fields 5 mm
+    into the arc; sigma in cells.  Returns the deposited J[comp] and the
+    oracle's in FP64 for the same (stored) particles."""
+    b = O.Bend(Nx=2200, Ny=240, **GEOM)
+    hx, hy = b.hr
+    phi0, c = 5e-3 / b.R, b.center
+    centre = np.array((c[0] + b.R * np.sin(phi0), c[1] - b.R * np.cos(phi0)))
+    th = phi0 + np.radians(tilt)
+    R, P, Q = gaussian_bunch(n, centre, sigma[0] * hx, sigma[1] * hy, 100.0, 1.0, seed=seed, energy_spread=1e-3,
+                             direction=(np.cos(th), np.sin(th)))
+    R = np.clip(R, centre - (190 * hx, 100 * hy), centre + (190 * hx, 100 * hy))
+    m = MovingWindowStep(512, 256, hx, hy, order=order, fp32=fp32, sortEvery=20, statModulus=0, **GEOM)
+    m.init_bunch(R, P, Q)
+    m.step(1)
+    inf = m.info()
+    (wx0, wy0), dt = inf["pos"], inf["dt"]
+    F = np.zeros((6, m.H + 2, m.W + 2))
+    F[0], F[1], F[2], F[3] = 2e7, -1e7, 1.5e7 / Z0, 1.5e7 / Z0
+    m.set_fields(F)
+    Fd = m.fields()
+    R0, P0 = m.particles()
+    origin = (inf["origin"][0] - hx, inf["origin"][1] - hy)
+    Rmid = O.push_patch(order, b, dt, Fd[0], Fd[1], Fd[2] + Fd[3], origin, (hx, hy), R0, P0, s2bug=False)[3]
+    m.push(comp)
+    J = m.fields()[4 + comp][1:-1, 1:-1]
+    m.close()
+    return J, O.deposit(order, comp, (wx0, wy0, m.W, m.H), tuple(b.origin), (hx, hy), dt, R0, Rmid, np.full(n, Q[0]))
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("fp32,n,sigma", [
+    (True, 1, (20, 10)), (True, 63, (20, 10)), (True, 257, (20, 10)), (True, 1025, (1, 1)), (True, 3001, (0.3, 0.3)),
+    (True, 340001, (20, 10)), (False, 65, (20, 10)), (False, 2049, (0.3, 0.3))])
+def test_sorted_push_forms_vs_oracle(gpu, fp32, n, sigma, order):
+    """The current of sorted particles: one per thread in workgroups of 256 up
+    to 200 particles per cell, of 1024 above (FP32); counts around a wavefront
+    and a workgroup, quads that share an anchor and quads that do not (at a
+    tilt).  FP32 as in test_production_push_vs_oracle; FP64 sums, 1e-11 of the
+    largest node."""
+    for comp, tilt in ((0, 0.0), (1, 25.0)):
+        J, Jo = sorted_push(order, fp32, n, sigma, comp, seed=n + order, tilt=tilt)
+        err = np.abs(J - Jo).max() / np.abs(Jo).max()
+        print("order %d, %d particles, sigma %g x %g, J[%d]: %.2e" % ((order, n) + sigma + (comp, err)))
+        assert err < (2e-5 if fp32 else 1e-11)
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("n,sigma", [(100000, (20, 10)), (300000, (20, 10)), (100000, (4, 4)), (100000, (1, 1))])
+def test_fp32_current_sums(gpu, order, n, sigma):
+    """The FP32 current of few particles is summed in FP64 within a workgroup,
+    so its error is that of the workgroups' additions to a node in FP32: G
+    additions of growing sums give 2^-25 sqrt(G / 3) of the node, the
+    particles' own roundings and the result's add 2^-25.  Workgroups are 256 or
+    (above 200 particles per cell) 1024 particles in sort order; a node's
+    stencil holds (order + 1)(order + 2) cells' particles, in workgroups
+    besides those that only touch it (4), and no more than there are.  A factor
+    1.5 over the root mean square of three bunches."""
+    per = n / (2 * np.pi * sigma[0] * sigma[1])
+    wg = 256 if per <= 200 else 1024
+    G = min((order + 1) * (order + 2) * per / wg + 4, np.ceil(n / wg))
+    sq = 0.0
+    for seed in range(3):
+        J, Jo = sorted_push(order, True, n, sigma, 0, seed=100 * seed + order)
+        sq += np.sum((J - Jo) ** 2) / np.sum(Jo ** 2) / 3
+    tol = 1.5 * 2.0 ** -25 * (1 + np.sqrt(G / 3))
+    print("order %d, %d particles, sigma %g x %g: L2 error %.2e (bound %.2e)" % ((order, n) + sigma + (np.sqrt(sq), tol)))
+    assert np.sqrt(sq) < tol
+
+
 def test_line_fields_vs_oracle(gpu):
     """SaveEMFieldsCommand (SaveEMFields.cpp:34-160) through csrst_line_fields
     after 40 steps into the bend and the copy of the window's E and H that
