@@ -34,10 +34,13 @@ constexpr int kNu = 2;             // sweeps before and after the coarse correct
 constexpr int kCoarseSweeps = 8;   // most sweeps on the coarsest level
 constexpr int kMaxTab = 32;        // run starts with a factor table of their own
 // Levels of at most this many nodes run in one workgroup (k_tail), where a
-// barrier replaces a launch.  One CU moves 64 B a cycle and a half sweep is
-// 16 B a node, so at this size the two cost the same, 3.3 us; below it the
-// workgroup wins.
-constexpr int kTailNodes = 16384;
+// barrier replaces a launch, but one CU's loads have to bring 32 B a node and
+// half sweep, and a wave solves several columns in turn.  us per V-cycle with
+// 2048, 4096, 8192, 16384 nodes: 512 x 256 243, 207, 212, 281; 1024 x 512 266,
+// 264, 264, 327; 2000 x 64 195, 224, 302, 497; 300 x 100 174, 188, 229, 319;
+// 100 x 2000 332, 325, 325, 340; 2048 x 1024 405, 411, 404, 438.  Without the
+// tail 64 x 48 takes 246 and 2000 x 64 258, with it 131 and 224.
+constexpr int kTailNodes = 4096;
 // Coarsening ends once a red/black sweep damps the smoothest error by this
 // factor: the x coupling is then weak against the line's own smallest
 // eigenvalue, and coarser levels would add launches only.
