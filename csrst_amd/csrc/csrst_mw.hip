@@ -750,257 +750,254 @@ __global__ void __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(1, NB >
 #pragma unroll
         for (int t = 0; t < NN; ++t) sacc[q][t] = T(0);
     }
+    const int k0 = kt;
+    int GX[PPT], GY[PPT];
+    T FX[PPT], FY[PPT], PX[PPT], PY[PPT];
+    load_run(p.gx, k0, p.n, GX);
+    load_run(p.gy, k0, p.n, GY);
+    load_run(p.fx, k0, p.n, FX);
+    load_run(p.fy, k0, p.n, FY);
+    load_run(p.px, k0, p.n, PX);
+    load_run(p.py, k0, p.n, PY);
 #pragma unroll 1
-    for (int r = 0; r < 1; ++r) {
-        const int k0 = kt;
-        int GX[PPT], GY[PPT];
-        T FX[PPT], FY[PPT], PX[PPT], PY[PPT];
-        load_run(p.gx, k0, p.n, GX);
-        load_run(p.gy, k0, p.n, GY);
-        load_run(p.fx, k0, p.n, FX);
-        load_run(p.fy, k0, p.n, FY);
-        load_run(p.px, k0, p.n, PX);
-        load_run(p.py, k0, p.n, PY);
-#pragma unroll 1
-        for (int u = 0; u < PPT; ++u) {
-            const bool live = k0 + u < p.n;
-            const int gx0 = GX[0], gy0 = GY[0];
-            const T fx0 = FX[0], fy0 = FY[0];
-            vec2<T> dP = pm::mk(PX[0], PY[0]), P = dP;
-            int gx = gx0, gy = gy0;
-            T fx = fx0, fy = fy0;
-            T g2 = 0;
-            T x1 = fx0, y1 = fy0, x2 = fx0, y2 = fy0;
-            if (live) {
-                P = pm::mk(p0.x + dP.x, p0.y + dP.y);
-                // half drift (PartBunch.cpp:228-232)
-                const T gi = pm::inv_gamma(P);
-                x1 = fx0 + c.hx * P.x * gi;
-                y1 = fy0 + c.hy * P.y * gi;
-                {
-                    const T flx = pm::floor_(x1), fly = pm::floor_(y1);
-                    gx = gx0 + (int)flx; gy = gy0 + (int)fly;
-                    fx = x1 - flx; fy = y1 - fly;
-                }
-                // gather at R1 (positions relative to the particle's cell corner).
-                // With fx, fy in [0, 1) every stencil of the three fields starts at
-                // node offset L or L + 1 from the cell and spans N nodes, so the
-                // ring-wrapped byte offsets of the U = N + 1 union columns and rows
-                // are formed once and each load is plane + row + column (32-bit
-                // offsets from the uniform plane base).
-                const vec2<T> pp = pm::mk(fx, fy);
-                constexpr int N = ORDER + 2, L = ORDER == 2 ? -2 : -1, U = N + 1;
-                // The union's first column and row, clamped so that all U
-                // stay inside the guarded window (a particle outside it has
-                // set the error bit; its loads stay in bounds), then the ring
-                // offsets: rows one by one (each may wrap), columns as one
-                // base when the U columns do not cross the ring's seam, so a
-                // row's loads take immediate offsets from one address.
-                uint32_t R[U], C0;
-                bool cwrap;
-                {
-                    const int i0 = gx + L - wx0, j0 = gy + L - wy0;
-                    if (i0 < -G || i0 + U - 1 > W - 1 + G || j0 < -G || j0 + U - 1 > H - 1 + G) err |= 1;
-                    int px = min(max(i0, -G), W - U + G) + G + rx;
-                    px = px >= f.Wp ? px - f.Wp : px;
-                    cwrap = px > f.Wp - U;
-                    C0 = (uint32_t)px * (uint32_t)sizeof(T);
-                    int py = min(max(j0, -G), H - U + G) + G + ry;
-                    py = py >= f.Hp ? py - f.Hp : py;
-                    const uint32_t rowb = (uint32_t)(f.Wp * sizeof(T));
-                    R[0] = (uint32_t)py * rowb;
-#pragma unroll
-                    for (int a = 1; a < U; ++a) {
-                        const bool wrap = ++py == f.Hp;
-                        py = wrap ? 0 : py;
-                        R[a] = wrap ? 0u : R[a - 1] + rowb;
-                    }
-                }
-                const bool anyWrap = __any(cwrap);
-                auto gat = [&](const T *plane, const pm::Stencil<T> &st) -> T {
-                    const bool sx = st.I0 != L, sy = st.J0 != L;
-                    uint32_t rr[N];
-#pragma unroll
-                    for (int a = 0; a < N; ++a) rr[a] = sy ? R[a + 1] : R[a];
-                    // The empty asm makes the plane pointer opaque here, so the
-                    // resource (four scalar registers) is built at each gather
-                    // instead of three being hoisted out of the particle loop,
-                    // where they push other scalars into spills (each reload
-                    // is a VALU readlane).
-                    const T *pl = plane;
-                    asm volatile("" : "+s"(pl));
-                    const auto rs = plane_rsrc(pl, f.plane);
-                    if (!anyWrap) {
-                        // one offset per row; its N columns are consecutive
-                        // (immediate offsets, merged into wide loads)
-                        const uint32_t cb = C0 + (sx ? (uint32_t)sizeof(T) : 0u);
-                        return pm::gather_n<N>(st, false, [&](int a, int b) {
-                            return buf_load<T>(rs, rr[b] + cb + (uint32_t)(a * sizeof(T)));
-                        });
-                    }
-                    // a stencil of this wavefront crosses the seam: per-column offsets
-                    uint32_t cc[N];
-                    {
-                        int px = (int)(C0 / (uint32_t)sizeof(T)) + (sx ? 1 : 0);
-#pragma unroll
-                        for (int a = 0; a < N; ++a) {
-                            px = px >= f.Wp ? px - f.Wp : px;
-                            cc[a] = (uint32_t)px * (uint32_t)sizeof(T);
-                            ++px;
-                        }
-                    }
-                    return pm::gather_n<N>(st, false, [&](int a, int b) { return buf_load<T>(rs, rr[b] + cc[a]); });
-                };
-                T ex, ey, hf;
-                if constexpr (ORDER == 2) {
-                    // The three S2 stencils use two weight sets per axis: at the
-                    // offset from the cell corner (Ex's y, Ey's x) and from the
-                    // nearest cell centre (Ex's x, Ey's y, both of Hz's)
-                    // (ScatterGatherImpl.hh:424-447, 486-505 with fx, fy in [0, 1)).
-                    pm::Stencil<T> sx, sy;
-                    const int lx = (int)pm::floor_(pp.x - T(0.5)), ly = (int)pm::floor_(pp.y - T(0.5));
-                    T wxu[4], wyu[4];
-                    s2_weights(pp.x - ((T)lx + T(0.5)), sx.wx);
-                    s2_weights(pp.y - ((T)ly + T(0.5)), sy.wy);
-                    s2_weights(pp.x, wxu);
-                    s2_weights(pp.y, wyu);
-                    pm::Stencil<T> st;
-                    st.n = 4;
-                    st.I0 = lx - 1; st.J0 = -1;
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) { st.wx[a] = sx.wx[a]; st.wy[a] = wyu[a]; }
-                    ex = gat(f.ex, st);
-                    st.I0 = -1; st.J0 = ly - 1;
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) { st.wx[a] = wxu[a]; st.wy[a] = sy.wy[a]; }
-                    ey = gat(f.ey, st);
-                    st.I0 = lx - 1;
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) st.wx[a] = sx.wx[a];
-                    hf = gat(f.hz, st);
-                } else {
-                    ex = gat(f.ex, pm::edge_stencil(ORDER, 0, pp));
-                    ey = gat(f.ey, pm::edge_stencil(ORDER, 1, pp));
-                    hf = gat(f.hz, pm::cell_stencil(ORDER, pp));
-                }
-                const double X = g.org[0] + ((double)gx + (double)fx) * g.h[0];
-                const double Y = g.org[1] + ((double)gy + (double)fy) * g.h[1];
-                const T bext = (T)geom::external_bz(g.bend, X, Y);
-                dP = kick_rotate_split(p0, dP, ex, ey, hf, bext, c.fact1, c.fact2);
-                P = pm::mk(p0.x + dP.x, p0.y + dP.y);
-                g2 = pm::inv_gamma(P);
-                x2 = x1 + c.hx * P.x * g2;
-                y2 = y1 + c.hy * P.y * g2;
+    for (int u = 0; u < PPT; ++u) {
+        const bool live = k0 + u < p.n;
+        const int gx0 = GX[0], gy0 = GY[0];
+        const T fx0 = FX[0], fy0 = FY[0];
+        vec2<T> dP = pm::mk(PX[0], PY[0]), P = dP;
+        int gx = gx0, gy = gy0;
+        T fx = fx0, fy = fy0;
+        T g2 = 0;
+        T x1 = fx0, y1 = fy0, x2 = fx0, y2 = fy0;
+        if (live) {
+            P = pm::mk(p0.x + dP.x, p0.y + dP.y);
+            // half drift (PartBunch.cpp:228-232)
+            const T gi = pm::inv_gamma(P);
+            x1 = fx0 + c.hx * P.x * gi;
+            y1 = fy0 + c.hy * P.y * gi;
+            {
+                const T flx = pm::floor_(x1), fly = pm::floor_(y1);
+                gx = gx0 + (int)flx; gy = gy0 + (int)fly;
+                fx = x1 - flx; fy = y1 - fly;
             }
-            // ---- deposit of R0 -> R2, cell units relative to the old cell corner
-            const vec2<T> o = pm::mk(fx0, fy0);
-            const vec2<T> e = pm::mk(x2, y2);
-            Split<T> xs;
-            const bool oneCross = split_path(xs, o, e, ORDER == 1);   // dead lanes: o = e = 0
-            if (live && !oneCross) err |= 2;
-            const vec2<T> delta = pm::mk(e.x - o.x, e.y - o.y);
-            const int nseg = live ? xs.n - 1 : 0;
-            if constexpr (PPT == 1) {
-#pragma unroll 1
-                for (int s = 0; s < 3; ++s) {
-                    const bool act = s < nseg;
-                    if (!__any(act)) break;
-                    pm::SegCurrent<T> sc;
-                    const vec2<T> xi = sel(s == 0, xs.s[0], sel(s == 1, xs.s[1], xs.s[2]));
-                    const vec2<T> xf = sel(s == 0, xs.s[1], sel(s == 1, xs.s[2], xs.s[3]));
-                    const T tau = s == 0 ? xs.f[1] - xs.f[0] : s == 1 ? xs.f[2] - xs.f[1] : xs.f[3] - xs.f[2];
-                    seg_current(sc, xi, xf, tau, delta, gx0, gy0);
-                    // one add per quad whose lanes share an anchor, else one per lane
-                    const int aI = sc.I0, aJ = act ? sc.J0 : INT_MIN + lane;
-                    const bool one = aI == dpp_i<0xb1, 0xf>(0, aI) && aJ == dpp_i<0xb1, 0xf>(0, aJ) &&
-                                     aI == dpp_i<0x4e, 0xf>(0, aI) && aJ == dpp_i<0x4e, 0xf>(0, aJ) &&
-                                     aI == dpp_i<0x1b, 0xf>(0, aI) && aJ == dpp_i<0x1b, 0xf>(0, aJ);
+            // gather at R1 (positions relative to the particle's cell corner).
+            // With fx, fy in [0, 1) every stencil of the three fields starts at
+            // node offset L or L + 1 from the cell and spans N nodes, so the
+            // ring-wrapped byte offsets of the U = N + 1 union columns and rows
+            // are formed once and each load is plane + row + column (32-bit
+            // offsets from the uniform plane base).
+            const vec2<T> pp = pm::mk(fx, fy);
+            constexpr int N = ORDER + 2, L = ORDER == 2 ? -2 : -1, U = N + 1;
+            // The union's first column and row, clamped so that all U
+            // stay inside the guarded window (a particle outside it has
+            // set the error bit; its loads stay in bounds), then the ring
+            // offsets: rows one by one (each may wrap), columns as one
+            // base when the U columns do not cross the ring's seam, so a
+            // row's loads take immediate offsets from one address.
+            uint32_t R[U], C0;
+            bool cwrap;
+            {
+                const int i0 = gx + L - wx0, j0 = gy + L - wy0;
+                if (i0 < -G || i0 + U - 1 > W - 1 + G || j0 < -G || j0 + U - 1 > H - 1 + G) err |= 1;
+                int px = min(max(i0, -G), W - U + G) + G + rx;
+                px = px >= f.Wp ? px - f.Wp : px;
+                cwrap = px > f.Wp - U;
+                C0 = (uint32_t)px * (uint32_t)sizeof(T);
+                int py = min(max(j0, -G), H - U + G) + G + ry;
+                py = py >= f.Hp ? py - f.Hp : py;
+                const uint32_t rowb = (uint32_t)(f.Wp * sizeof(T));
+                R[0] = (uint32_t)py * rowb;
 #pragma unroll
-                    for (int t = 0; t < NN; ++t) {
-                        const T q = quad_sum(sc.w[t]);
-                        sc.w[t] = one ? q : sc.w[t];
-                    }
-                    if (act && (!one || (lane & 3) == 0)) lane_add(sc.I0, sc.J0, sc.w);
+                for (int a = 1; a < U; ++a) {
+                    const bool wrap = ++py == f.Hp;
+                    py = wrap ? 0 : py;
+                    R[a] = wrap ? 0u : R[a - 1] + rowb;
                 }
+            }
+            const bool anyWrap = __any(cwrap);
+            auto gat = [&](const T *plane, const pm::Stencil<T> &st) -> T {
+                const bool sx = st.I0 != L, sy = st.J0 != L;
+                uint32_t rr[N];
+#pragma unroll
+                for (int a = 0; a < N; ++a) rr[a] = sy ? R[a + 1] : R[a];
+                // The empty asm makes the plane pointer opaque here, so the
+                // resource (four scalar registers) is built at each gather
+                // instead of three being hoisted out of the particle loop,
+                // where they push other scalars into spills (each reload
+                // is a VALU readlane).
+                const T *pl = plane;
+                asm volatile("" : "+s"(pl));
+                const auto rs = plane_rsrc(pl, f.plane);
+                if (!anyWrap) {
+                    // one offset per row; its N columns are consecutive
+                    // (immediate offsets, merged into wide loads)
+                    const uint32_t cb = C0 + (sx ? (uint32_t)sizeof(T) : 0u);
+                    return pm::gather_n<N>(st, false, [&](int a, int b) {
+                        return buf_load<T>(rs, rr[b] + cb + (uint32_t)(a * sizeof(T)));
+                    });
+                }
+                // a stencil of this wavefront crosses the seam: per-column offsets
+                uint32_t cc[N];
+                {
+                    int px = (int)(C0 / (uint32_t)sizeof(T)) + (sx ? 1 : 0);
+#pragma unroll
+                    for (int a = 0; a < N; ++a) {
+                        px = px >= f.Wp ? px - f.Wp : px;
+                        cc[a] = (uint32_t)px * (uint32_t)sizeof(T);
+                        ++px;
+                    }
+                }
+                return pm::gather_n<N>(st, false, [&](int a, int b) { return buf_load<T>(rs, rr[b] + cc[a]); });
+            };
+            T ex, ey, hf;
+            if constexpr (ORDER == 2) {
+                // The three S2 stencils use two weight sets per axis: at the
+                // offset from the cell corner (Ex's y, Ey's x) and from the
+                // nearest cell centre (Ex's x, Ey's y, both of Hz's)
+                // (ScatterGatherImpl.hh:424-447, 486-505 with fx, fy in [0, 1)).
+                pm::Stencil<T> sx, sy;
+                const int lx = (int)pm::floor_(pp.x - T(0.5)), ly = (int)pm::floor_(pp.y - T(0.5));
+                T wxu[4], wyu[4];
+                s2_weights(pp.x - ((T)lx + T(0.5)), sx.wx);
+                s2_weights(pp.y - ((T)ly + T(0.5)), sy.wy);
+                s2_weights(pp.x, wxu);
+                s2_weights(pp.y, wyu);
+                pm::Stencil<T> st;
+                st.n = 4;
+                st.I0 = lx - 1; st.J0 = -1;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) { st.wx[a] = sx.wx[a]; st.wy[a] = wyu[a]; }
+                ex = gat(f.ex, st);
+                st.I0 = -1; st.J0 = ly - 1;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) { st.wx[a] = wxu[a]; st.wy[a] = sy.wy[a]; }
+                ey = gat(f.ey, st);
+                st.I0 = lx - 1;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) st.wx[a] = sx.wx[a];
+                hf = gat(f.hz, st);
             } else {
-            // third segments (a push crossing a cell column and a cell row) are
-            // queued and computed 64 at a time: in-line, one lane with three
-            // segments makes its whole wavefront run a third segment pass
-            const bool has3 = nseg == 3;
-            const unsigned long long m3 = __ballot(has3);
-            if (m3) {
-                const int cnt = __popcll(m3);
-                if (qn + cnt > 64) drain_queue();
-                if (has3) {
-                    const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m3 >> 32),
-                                                                       __builtin_amdgcn_mbcnt_lo((unsigned)m3, 0u));
-                    qv[0][at] = xs.s[2].x; qv[1][at] = xs.s[2].y;
-                    qv[2][at] = xs.s[3].x; qv[3][at] = xs.s[3].y;
-                    qv[4][at] = xs.f[3] - xs.f[2];
-                    qv[5][at] = delta.x; qv[6][at] = delta.y;
-                    qg[0][at] = gx0; qg[1][at] = gy0;
-                }
-                qn += cnt;
+                ex = gat(f.ex, pm::edge_stencil(ORDER, 0, pp));
+                ey = gat(f.ey, pm::edge_stencil(ORDER, 1, pp));
+                hf = gat(f.hz, pm::cell_stencil(ORDER, pp));
             }
+            const double X = g.org[0] + ((double)gx + (double)fx) * g.h[0];
+            const double Y = g.org[1] + ((double)gy + (double)fy) * g.h[1];
+            const T bext = (T)geom::external_bz(g.bend, X, Y);
+            dP = kick_rotate_split(p0, dP, ex, ey, hf, bext, c.fact1, c.fact2);
+            P = pm::mk(p0.x + dP.x, p0.y + dP.y);
+            g2 = pm::inv_gamma(P);
+            x2 = x1 + c.hx * P.x * g2;
+            y2 = y1 + c.hy * P.y * g2;
+        }
+        // ---- deposit of R0 -> R2, cell units relative to the old cell corner
+        const vec2<T> o = pm::mk(fx0, fy0);
+        const vec2<T> e = pm::mk(x2, y2);
+        Split<T> xs;
+        const bool oneCross = split_path(xs, o, e, ORDER == 1);   // dead lanes: o = e = 0
+        if (live && !oneCross) err |= 2;
+        const vec2<T> delta = pm::mk(e.x - o.x, e.y - o.y);
+        const int nseg = live ? xs.n - 1 : 0;
+        if constexpr (PPT == 1) {
 #pragma unroll 1
-            for (int s = 0; s < 2; ++s) {
+            for (int s = 0; s < 3; ++s) {
                 const bool act = s < nseg;
                 if (!__any(act)) break;
                 pm::SegCurrent<T> sc;
-                {
-                    // slot selects instead of xs.s[s] keep the list in registers
-                    const vec2<T> xi = sel(s == 0, xs.s[0], xs.s[1]);
-                    const vec2<T> xf = sel(s == 0, xs.s[1], xs.s[2]);
-                    const T tau = s == 0 ? xs.f[1] - xs.f[0] : xs.f[2] - xs.f[1];
-                    seg_current(sc, xi, xf, tau, delta, gx0, gy0);
-                }
-                // register accumulation by anchor: the first kSlots anchors a
-                // lane meets own its slots, in order (their sums start at
-                // zero); a segment matching none goes to the LDS tile
-                // (MISSCOOP: through the wavefront).  Independent conditional
-                // adds: a wavefront whose lanes take different slots pays one
-                // pass per slot taken.
-                bool taken = !act;
+                const vec2<T> xi = sel(s == 0, xs.s[0], sel(s == 1, xs.s[1], xs.s[2]));
+                const vec2<T> xf = sel(s == 0, xs.s[1], sel(s == 1, xs.s[2], xs.s[3]));
+                const T tau = s == 0 ? xs.f[1] - xs.f[0] : s == 1 ? xs.f[2] - xs.f[1] : xs.f[3] - xs.f[2];
+                seg_current(sc, xi, xf, tau, delta, gx0, gy0);
+                // one add per quad whose lanes share an anchor, else one per lane
+                const int aI = sc.I0, aJ = act ? sc.J0 : INT_MIN + lane;
+                const bool one = aI == dpp_i<0xb1, 0xf>(0, aI) && aJ == dpp_i<0xb1, 0xf>(0, aJ) &&
+                                 aI == dpp_i<0x4e, 0xf>(0, aI) && aJ == dpp_i<0x4e, 0xf>(0, aJ) &&
+                                 aI == dpp_i<0x1b, 0xf>(0, aI) && aJ == dpp_i<0x1b, 0xf>(0, aJ);
 #pragma unroll
-                for (int q = 0; q < kSlots; ++q) {
-                    const bool to = !taken && (!has[q] || (sc.I0 == sI[q] && sc.J0 == sJ[q]));
-                    sI[q] = to ? sc.I0 : sI[q];
-                    sJ[q] = to ? sc.J0 : sJ[q];
-                    has[q] = has[q] || to;
-                    if (to) {
-#pragma unroll
-                        for (int t = 0; t < NN; ++t) sacc[q][t] += sc.w[t];
-                    }
-                    taken = taken || to;
+                for (int t = 0; t < NN; ++t) {
+                    const T q = quad_sum(sc.w[t]);
+                    sc.w[t] = one ? q : sc.w[t];
                 }
-                const bool miss = !taken;
-                if (MISSCOOP) {
-                    if (__any(miss)) coop_add(miss, sc.I0, sc.J0, sc.w);
-                } else if (miss) {
-                    lane_add(sc.I0, sc.J0, sc.w);
-                }
+                if (act && (!one || (lane & 3) == 0)) lane_add(sc.I0, sc.J0, sc.w);
             }
+        } else {
+        // third segments (a push crossing a cell column and a cell row) are
+        // queued and computed 64 at a time: in-line, one lane with three
+        // segments makes its whole wavefront run a third segment pass
+        const bool has3 = nseg == 3;
+        const unsigned long long m3 = __ballot(has3);
+        if (m3) {
+            const int cnt = __popcll(m3);
+            if (qn + cnt > 64) drain_queue();
+            if (has3) {
+                const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m3 >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m3, 0u));
+                qv[0][at] = xs.s[2].x; qv[1][at] = xs.s[2].y;
+                qv[2][at] = xs.s[3].x; qv[3][at] = xs.s[3].y;
+                qv[4][at] = xs.f[3] - xs.f[2];
+                qv[5][at] = delta.x; qv[6][at] = delta.y;
+                qg[0][at] = gx0; qg[1][at] = gy0;
             }
-            // ---- drift back by half a step (TETMSolver.hh:210, 265)
-            if (live) {
-                const int ex2 = gx0 + (int)pm::floor_(x2), ey2 = gy0 + (int)pm::floor_(y2);
-                bminx = min(bminx, min(gx0, ex2)); bminy = min(bminy, min(gy0, ey2));
-                bmaxx = max(bmaxx, max(gx0, ex2)); bmaxy = max(bmaxy, max(gy0, ey2));
-                gx = gx0; gy = gy0; fx = T(0); fy = T(0);
-                split_add(gx, fx, x2 - c.hx * P.x * g2);
-                split_add(gy, fy, y2 - c.hy * P.y * g2);
-            }
-            rotate_in(GX, gx); rotate_in(GY, gy);
-            rotate_in(FX, fx); rotate_in(FY, fy);
-            rotate_in(PX, dP.x); rotate_in(PY, dP.y);
+            qn += cnt;
         }
-        store_run(p.gx, k0, p.n, GX);
-        store_run(p.gy, k0, p.n, GY);
-        store_run(p.fx, k0, p.n, FX);
-        store_run(p.fy, k0, p.n, FY);
-        store_run(p.px, k0, p.n, PX);
-        store_run(p.py, k0, p.n, PY);
+#pragma unroll 1
+        for (int s = 0; s < 2; ++s) {
+            const bool act = s < nseg;
+            if (!__any(act)) break;
+            pm::SegCurrent<T> sc;
+            {
+                // slot selects instead of xs.s[s] keep the list in registers
+                const vec2<T> xi = sel(s == 0, xs.s[0], xs.s[1]);
+                const vec2<T> xf = sel(s == 0, xs.s[1], xs.s[2]);
+                const T tau = s == 0 ? xs.f[1] - xs.f[0] : xs.f[2] - xs.f[1];
+                seg_current(sc, xi, xf, tau, delta, gx0, gy0);
+            }
+            // register accumulation by anchor: the first kSlots anchors a
+            // lane meets own its slots, in order (their sums start at
+            // zero); a segment matching none goes to the LDS tile
+            // (MISSCOOP: through the wavefront).  Independent conditional
+            // adds: a wavefront whose lanes take different slots pays one
+            // pass per slot taken.
+            bool taken = !act;
+#pragma unroll
+            for (int q = 0; q < kSlots; ++q) {
+                const bool to = !taken && (!has[q] || (sc.I0 == sI[q] && sc.J0 == sJ[q]));
+                sI[q] = to ? sc.I0 : sI[q];
+                sJ[q] = to ? sc.J0 : sJ[q];
+                has[q] = has[q] || to;
+                if (to) {
+#pragma unroll
+                    for (int t = 0; t < NN; ++t) sacc[q][t] += sc.w[t];
+                }
+                taken = taken || to;
+            }
+            const bool miss = !taken;
+            if (MISSCOOP) {
+                if (__any(miss)) coop_add(miss, sc.I0, sc.J0, sc.w);
+            } else if (miss) {
+                lane_add(sc.I0, sc.J0, sc.w);
+            }
+        }
+        }
+        // ---- drift back by half a step (TETMSolver.hh:210, 265)
+        if (live) {
+            const int ex2 = gx0 + (int)pm::floor_(x2), ey2 = gy0 + (int)pm::floor_(y2);
+            bminx = min(bminx, min(gx0, ex2)); bminy = min(bminy, min(gy0, ey2));
+            bmaxx = max(bmaxx, max(gx0, ex2)); bmaxy = max(bmaxy, max(gy0, ey2));
+            gx = gx0; gy = gy0; fx = T(0); fy = T(0);
+            split_add(gx, fx, x2 - c.hx * P.x * g2);
+            split_add(gy, fy, y2 - c.hy * P.y * g2);
+        }
+        rotate_in(GX, gx); rotate_in(GY, gy);
+        rotate_in(FX, fx); rotate_in(FY, fy);
+        rotate_in(PX, dP.x); rotate_in(PY, dP.y);
     }
+    store_run(p.gx, k0, p.n, GX);
+    store_run(p.gy, k0, p.n, GY);
+    store_run(p.fx, k0, p.n, FX);
+    store_run(p.fy, k0, p.n, FY);
+    store_run(p.px, k0, p.n, PX);
+    store_run(p.py, k0, p.n, PY);
     // ---- queued third segments, then the register slots
     if constexpr (PPT > 1) {
     if (qn) drain_queue();
@@ -2088,7 +2085,7 @@ void one_step(csrst_mw *m, bool timed)
     constexpr int kW = mw::kB / 64;
     auto waves = [](int n, int per) { return (n + per - 1) / per; };
     // the sweep: interior columns (and, without layers, the guard columns) by
-    // strips; the layers' waves in extra rows of the grid
+    // strips, after the layers' workgroups
     const int cols = np ? W - 2 * np : W + 1, gx = waves(waves(cols, mw::kCols), kW);
     const int pmlBlocks = np ? (waves(waves(2 * np + 2, 64) * waves(H, mw::kPmlStrip), kW) + 7) & ~7 : 0;
     const int gs = pmlBlocks + gx * waves(H, mw::kStrip);
