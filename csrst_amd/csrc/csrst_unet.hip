@@ -1250,10 +1250,14 @@ void plan(csrst_warmstart *u, int B)
     u->batch = B;
 }
 
+// the activations (of plan) that each convolution reads and writes
+constexpr int kConvs = 15;
+constexpr int kIn[kConvs] = {0, 1, 3, 4, 6, 7, 9, 10, 11, 13, 14, 16, 17, 19, 20};
+constexpr int kOut[kConvs] = {1, 2, 4, 5, 7, 8, 10, 11, 12, 14, 15, 17, 18, 20, 21};
+
 void forward(csrst_warmstart *u, int B)
 {
     auto &A = u->A;
-    const int H = u->H, W = u->W;
     auto P = [&](int i) { return u->ptr(A[i]); };
     auto pool = [&](int src, int dst) {
         const auto &d = A[dst];
@@ -1263,27 +1267,31 @@ void forward(csrst_warmstart *u, int B)
         const auto &d = A[dst];
         k_up_add<<<nb((size_t)B * d.h * d.w * d.c / 8), kB, 0, u->s>>>(P(src), P(skip), P(dst), B, d.h, d.w, d.c);
     };
-    conv(u, 0, P(0), P(1), nullptr, B, H, W);
-    conv(u, 1, P(1), P(2), nullptr, B, H, W);
+    auto c = [&](int li) {
+        const auto &d = A[kOut[li]];
+        conv(u, li, P(kIn[li]), P(kOut[li]), li + 1 == kConvs ? u->outf.p : nullptr, B, d.h, d.w);
+    };
+    c(0);
+    c(1);
     pool(2, 3);
-    conv(u, 2, P(3), P(4), nullptr, B, H / 2, W / 2);
-    conv(u, 3, P(4), P(5), nullptr, B, H / 2, W / 2);
+    c(2);
+    c(3);
     pool(5, 6);
-    conv(u, 4, P(6), P(7), nullptr, B, H / 4, W / 4);
-    conv(u, 5, P(7), P(8), nullptr, B, H / 4, W / 4);
+    c(4);
+    c(5);
     pool(8, 9);
-    conv(u, 6, P(9), P(10), nullptr, B, H / 8, W / 8);
-    conv(u, 7, P(10), P(11), nullptr, B, H / 8, W / 8);
-    conv(u, 8, P(11), P(12), nullptr, B, H / 8, W / 8);
+    c(6);
+    c(7);
+    c(8);
     upadd(12, 8, 13);
-    conv(u, 9, P(13), P(14), nullptr, B, H / 4, W / 4);
-    conv(u, 10, P(14), P(15), nullptr, B, H / 4, W / 4);
+    c(9);
+    c(10);
     upadd(15, 5, 16);
-    conv(u, 11, P(16), P(17), nullptr, B, H / 2, W / 2);
-    conv(u, 12, P(17), P(18), nullptr, B, H / 2, W / 2);
+    c(11);
+    c(12);
     upadd(18, 2, 19);
-    conv(u, 13, P(19), P(20), nullptr, B, H, W);
-    conv(u, 14, P(20), P(21), u->outf.p, B, H, W);
+    c(13);
+    c(14);
     HU_LAUNCH_CHECK();
 }
 
@@ -1292,17 +1300,18 @@ void backward(csrst_warmstart *u, int B)
 {
     auto &A = u->A;
     auto &G = u->Gd;
-    const int H = u->H, W = u->W;
     auto P = [&](int i) { return u->ptr(A[i]); };
     auto D = [&](int i) { return u->ptr(G[i]); };
     HU_CHECK(hipMemsetAsync(u->g.p, 0, u->nparam * sizeof(float), u->s));
-    // conv li with input activation xin and output activation yout.  D(yout) is
-    // the gradient before the ReLU: whatever produces a gradient at a ReLU's
-    // output masks it there.
-    auto back = [&](int li, int xin, int yout, int h, int w, bool needDx) {
-        const bool relu = xin == 20 || xin == 17 || xin == 14 || xin == 11 || xin == 10 || xin == 7 || xin == 4 || xin == 1;
-        conv_wgrad(u, li, D(yout), P(xin), B, h, w);
-        if (needDx) conv_dgrad(u, li, D(yout), D(xin), relu ? P(xin) : nullptr, B, h, w);
+    // conv li, from D of its output to D of its input.  D of a ReLU's output is
+    // the gradient before the ReLU: whatever produces a gradient there masks it.
+    auto back = [&](int li) {
+        const int x = kIn[li], y = kOut[li];
+        const auto &d = A[y];
+        conv_wgrad(u, li, D(y), P(x), B, d.h, d.w);
+        if (li == 0) return;
+        const bool relu = x == kOut[li - 1] && u->L[li - 1].relu;   // not a pooled or upsampled sum
+        conv_dgrad(u, li, D(y), D(x), relu ? P(x) : nullptr, B, d.h, d.w);
     };
     auto upgrad = [&](int dstLow, int srcHigh) {      // D(dstLow) = up^T D(srcHigh)
         const auto &d = A[dstLow];
@@ -1312,27 +1321,27 @@ void backward(csrst_warmstart *u, int B)
         const auto &d = A[at];
         k_skip_grad<<<nb((size_t)B * d.h * d.w * d.c / 8), kB, 0, u->s>>>(D(low), D(dec), P(at), D(at), B, d.h, d.w, d.c);
     };
-    back(14, 20, 21, H, W, true);      // out -> D20
-    back(13, 19, 20, H, W, true);      // -> D19 (= d(up(c02)) and d(s0))
-    upgrad(18, 19);                    // D18 = up^T D19
-    back(12, 17, 18, H / 2, W / 2, true);
-    back(11, 16, 17, H / 2, W / 2, true);
+    back(14);             // out -> D20
+    back(13);             // -> D19 (= d(up(c02)) and d(s0))
+    upgrad(18, 19);       // D18 = up^T D19
+    back(12);
+    back(11);
     upgrad(15, 16);
-    back(10, 14, 15, H / 4, W / 4, true);
-    back(9, 13, 14, H / 4, W / 4, true);
+    back(10);
+    back(9);
     upgrad(12, 13);
-    back(8, 11, 12, H / 8, W / 8, true);
-    back(7, 10, 11, H / 8, W / 8, true);
-    back(6, 9, 10, H / 8, W / 8, true);
+    back(8);
+    back(7);
+    back(6);
     skipgrad(8, 9, 13);
-    back(5, 7, 8, H / 4, W / 4, true);
-    back(4, 6, 7, H / 4, W / 4, true);
+    back(5);
+    back(4);
     skipgrad(5, 6, 16);
-    back(3, 4, 5, H / 2, W / 2, true);
-    back(2, 3, 4, H / 2, W / 2, true);
+    back(3);
+    back(2);
     skipgrad(2, 3, 19);
-    back(1, 1, 2, H, W, true);
-    back(0, 0, 1, H, W, false);
+    back(1);
+    back(0);
     HU_LAUNCH_CHECK();
 }
 
