@@ -37,7 +37,6 @@
 #include "hip_util.h"
 #include "pic_math.h"
 
-using hu::DBuf;
 using hu::Error;
 using pm::vec2;
 

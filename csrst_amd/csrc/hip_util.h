@@ -131,7 +131,9 @@ public:
             }
         if (pin_) (void)hipHostFree(pin_);
     }
-    // dst (device) = src (host); src may be reused when the call returns
+    // dst (device) = src (host).  Pageable memory may be reused when the call
+    // returns; pinned memory only once the stream has been waited for, as the
+    // callers do before they return.
     void in(void *dst, const void *src, size_t bytes, hipStream_t s)
     {
         if (!staged(src, bytes)) {
