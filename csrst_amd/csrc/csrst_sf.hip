@@ -321,9 +321,17 @@ __global__ void __launch_bounds__(kB) k_node_scan(const int2 *at, const double *
     }
 }
 
-// The node scan reads every item once per node: up to this many it takes less
-// than the sort path's launches (about 45 us at the limit, against 150 us).
-bool node_scan_fits(size_t items, size_t nodes) { return items > 0 && nodes <= 130000000u / items; }
+// The node scan's time is a wave per node (0.17 ns a node, as long as 400 items
+// take) and every item once per node (0.3 to 0.6 ps each), and at least one
+// wave's walk over the items (0.7 us per 256).  us, scan / sort, S2 currents (4
+// items a particle) | S0 charges:
+//   32 x 32 nodes    n 128 23/69 | 17/27    n 8192 121/131 | 40/66     n 32768 376/319 | 101/86
+//   128 x 128        n 1   20/45 | 19/25    n 1024  62/93  | 27/41     n 8192  308/126 | 88/64
+//   512 x 512        n 1   66/47 | 59/27    n 128  102/74  | 60/29
+//   4096 x 4096      n 1 3100/69 | 2750/45
+// (the line lies where they cross, with the node's own cost taken high: a charge
+// of few particles on 300 x 300 nodes takes about as long either way).
+bool node_scan_fits(size_t items, size_t nodes) { return items > 0 && items <= 32768 && nodes <= 90000000u / (items + 1000); }
 
 // ---------------------------------------------------------------------------
 // Large deposits: contributions in order, sorted by node.

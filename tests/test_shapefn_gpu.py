@@ -8,6 +8,7 @@ checked against the discrete continuity equation with the GPU's own
 currents (dt div J = -(rho(R) - rho(oldR)) to round-off).
 """
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -96,10 +97,8 @@ def test_charge_diff_continuity(gpu, order):
 @pytest.mark.parametrize("order", [0, 1, 2])
 @pytest.mark.parametrize("n", [1, 63, 65, 20312, 20313, 60000])
 def test_small_and_sorted_deposits_bitwise(gpu, order, n):
-    """Particle counts around a wavefront, around the line between the node
-    scan and the sorted deposit (130e6 item-node pairs: 20312 trajectories on
-    40 x 40 nodes), and runs of hundreds of contributions per node; the
-    repeated call takes the first one's workspace."""
+    """Particle counts around a wavefront and above, and runs of hundreds of
+    contributions per node; the repeated call takes the first one's workspace."""
     dx, dt = (0.7, 1.3), 0.37
     box, org = (-6, -6, 40, 40), (0.0, 0.0)
     oldR, R, q = trajectories(n, order + n)
@@ -108,6 +107,40 @@ def test_small_and_sorted_deposits_bitwise(gpu, order, n):
         for _ in range(2):
             assert same(SF.getCurrentDensity(order, comp, box, org, dx, dt, oldR, R, q), ref), "comp %d" % comp
     assert same(SF.getChargeDensity(order, box, org, dx, R, q), O.charge_density(order, box, org, dx, R, q))
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("n,nx,ny", [(8192, 40, 40), (8193, 40, 40), (1, 300, 298), (1, 300, 300)])
+def test_deposits_at_the_node_scans_limits_bitwise(gpu, order, n, nx, ny):
+    """Both sides of the lines between the node scan and the sorted deposit:
+    32768 items (4 a trajectory), and the cost of the nodes themselves."""
+    dx, dt = (0.7, 1.3), 0.37
+    box, org = (-6, -6, nx, ny), (0.0, 0.0)
+    oldR, R, q = trajectories(n, order + n)
+    for comp in (0, 1):
+        assert same(SF.getCurrentDensity(order, comp, box, org, dx, dt, oldR, R, q),
+                    O.deposit(order, comp, box, org, dx, dt, oldR, R, q)), "comp %d" % comp
+
+
+def test_few_particles_on_a_large_patch(gpu):
+    """The time of one particle's charge on 4096 x 4096 nodes is that of the
+    cleared patch, as a thousand particles' is (a wave per node took 40 times as
+    long)."""
+    n, side = 1024, 4096
+    f = SF.DeviceArray(shape=(side * side,))
+    R, Q = SF.DeviceArray(host=np.random.default_rng(3).uniform(8, 4000, (n, 2))), SF.DeviceArray(host=np.ones(n))
+
+    def median(k):
+        t = []
+        for _ in range(15):
+            t0 = time.perf_counter()
+            check(gpu.csrst_sf_charge_density(C.c_int(1), f.ptr, C.c_int(0), C.c_int(0), C.c_int(side), C.c_int(side),
+                                              SF._v2((0, 0)), SF._v2((1, 1)), R.ptr, Q.ptr, C.c_int(k), None))
+            t.append(time.perf_counter() - t0)
+        return sorted(t)[7]
+
+    many = median(n)
+    assert median(1) <= 2 * many
 
 
 def test_patch_overflow_is_reported(gpu):
