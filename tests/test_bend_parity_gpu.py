@@ -245,12 +245,12 @@ def test_production_push_vs_oracle(gpu, fp32, comp, tilt):
 @pytest.mark.parametrize("fp32,n", [(True, 63), (True, 257), (True, 340001), (True, 1500001), (False, 999999),
                                     (False, 1000001)])
 def test_push_forms_vs_oracle(gpu, fp32, n, order):
-    """The push takes one particle per thread up to a count and a run of them
-    above (FP32: 1.5e6, 6.5e5 and 3.5e5 for the orders 0, 1, 2; FP64: 1e6):
-    either form on uniform fields against the oracle, in the bend and at a
-    tilt, with odd counts.  A node sums up to 3e4 contributions, whose FP32
-    rounding is sqrt(3e4) 2^-24 = 1e-5 of it; momenta and positions are single
-    particles', as in test_production_push_vs_oracle."""
+    """The push of particles that were never sorted, on uniform fields against
+    the oracle, in the bend and at a tilt, with odd counts: FP64 one particle
+    per thread up to 1e6 and a run of them above, FP32 a run of them (sorted
+    ones: test_sorted_push_forms_vs_oracle).  A node sums up to 3e4
+    contributions, whose FP32 rounding is sqrt(3e4) 2^-24 = 1e-5 of it; momenta
+    and positions are single particles', as in test_production_push_vs_oracle."""
     b = O.Bend(Nx=1100, Ny=120, **GEOM)
     hx, hy = b.hr
     R, P, Q = arc_bunch(n, 5e-3, 25.0, seed=n)
@@ -272,7 +272,7 @@ def test_push_forms_vs_oracle(gpu, fp32, n, order):
     err = (np.abs((P1 - P0) - (Po - P0)).max() / np.abs(Po - P0).max(), np.abs(R1 - Ro).max() / hx,
            np.abs(J - Jo).max() / np.abs(Jo).max())
     print("push %s order %d, %d particles: dP %.2e, R %.2e cells, J %.2e" % (("FP32" if fp32 else "FP64", order, n) + err))
-    tol = (2e-5, 2e-6, 5e-5) if fp32 else (1e-11, 1e-12, 1e-11)
+    tol = (2e-5, 2e-6, 2e-5) if fp32 else (1e-11, 1e-12, 1e-11)
     assert all(e < t for e, t in zip(err, tol)), err
 
 

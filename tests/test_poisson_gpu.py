@@ -60,7 +60,7 @@ def test_multigrid_rejects_bad_input(gpu):
 
 
 def test_multigrid_long_lines(gpu):
-    """Columns longer than the LDS line solver takes use the per-thread path."""
+    """Columns longer than a wave holds at once (2048 rows) are solved in chunks."""
     flag, active, b = masked_grid(24, 2600, 4)
     cls = P.classes(flag, active)
     phi, cyc, res = P.solve(50 * 2e-4, 2e-4, cls, b, tol=1e-12, maxit=60)
