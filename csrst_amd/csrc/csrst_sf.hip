@@ -381,10 +381,11 @@ __global__ void __launch_bounds__(1024) k_scan(int *sum, int m, int *total)
 }
 
 // Contributions of 64 particles per workgroup: key = the node's index in the
-// patch (kEmpty outside it), value = its weight.  cnt != null: packed, sum[b]
-// items before workgroup b's; else ITEMS fixed items per particle, unused ones
-// kEmpty.  The rows of an item pass through LDS, so that the workgroup writes
-// them along memory (a thread writing its own rows takes a cache line each).
+// patch (kEmpty outside it), value = its weight.  cnt != null: packed, cnt[k]
+// items of particle k, sum[b] before workgroup b's; else ITEMS fixed items per
+// particle, unused ones kEmpty.  The rows of an item pass through LDS, so that
+// the workgroup writes them along memory (a thread writing its own rows takes a
+// cache line each).
 template <class Op>
 __global__ void __launch_bounds__(64) k_emit(Op op, int n, const uint8_t *cnt, const int *sum, unsigned *key, double *val,
                                              int *flags)
@@ -401,14 +402,16 @@ __global__ void __launch_bounds__(64) k_emit(Op op, int n, const uint8_t *cnt, c
     if (items < 0) flags[1] = 1;
     items = max(items, 0);
     if (cnt) {
-        int x = items;
+        // the places are those counted, whatever the caller's arrays hold by now
+        const int places = k < n ? cnt[k] : 0;
+        int x = places;
         for (int o = 1; o < 64; o <<= 1) {
             const int y = __shfl_up(x, o, 64);
             if (tid >= o) x += y;
         }
-        first[tid] = sum[blockIdx.x] + x - items;
-        many[tid] = items;
-        most = items;
+        first[tid] = sum[blockIdx.x] + x - places;
+        many[tid] = places;
+        most = places;
         for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
     } else {
         first[tid] = k * Op::ITEMS;
