@@ -8,6 +8,7 @@ checked against the discrete continuity equation with the GPU's own
 currents (dt div J = -(rho(R) - rho(oldR)) to round-off).
 """
 import ctypes as C
+import threading
 import time
 
 import numpy as np
@@ -275,6 +276,36 @@ def test_charge_on_a_patch_wider_than_2_28(gpu):
     R = SF.DeviceArray(host=np.array([[nx - 1 + 0.25 + i0, 0.5], [3.2e8, 0.5]]))
     assert run() == -4
     assert [node(nx - 1, j) for j in (0, 1)] == [0.375, 0.375] and node(0, 1) == 0 and node(2 ** 28, 0) == 0
+
+
+def test_deposits_from_several_threads(gpu):
+    """Four threads, each on a stream of its own, with counts on both sides of
+    the sort: the shared workspaces never mix, bit for bit."""
+    dx, dt = (0.7, 1.3), 0.37
+    box, org = (-6, -6, 40, 40), (0.0, 0.0)
+    jobs = [(order, trajectories(n, order + n)) for order in (0, 1, 2) for n in (300, 9000, 30000)]
+    want = [O.deposit(order, 0, box, org, dx, dt, *t) for order, t in jobs]
+    bad = []
+
+    def work(first):
+        st = SF.Stream()
+        for r in range(3):
+            for k in range(len(jobs)):
+                k = (k * (first + 1) + r) % len(jobs)
+                order, t = jobs[k]
+                J, o, e, q = SF.DeviceArray(shape=box[2:]), *(SF.DeviceArray(host=a) for a in t)
+                rc = gpu.csrst_sf_current_density(C.c_int(order), C.c_int(0), J.ptr, *(C.c_int(v) for v in box), SF._v2(org),
+                                                  SF._v2(dx), C.c_double(dt), o.ptr, e.ptr, q.ptr, C.c_int(len(t[2])), st.h)
+                if rc != 0 or not same(J.get(), want[k]):
+                    bad.append((first, r, k))
+        st.close()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
 
 
 def free_bytes():
